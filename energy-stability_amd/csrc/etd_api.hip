@@ -232,6 +232,19 @@ extern "C" int etd_create(const etd_params *p, const double *Vh, const double *V
     arrange_A(n, c->hV, h4, MT, nkc);
     HCHK(c, hipMemcpy(c->V4, h4, sizeof(double) * a4n, hipMemcpyHostToDevice));
     free(h4);
+    if (fold_parity(n, c->hVi, 1, &c->Vif_e0) && fold_parity(n, c->hV, 0, &c->Vf_e0)) {
+      const size_t afn = fold_A_doubles(n);
+      double *hf = (double *)malloc(sizeof(double) * afn);
+      if (!hf) return seterr(c, ETD_ERR_NOMEM, "folded basis");
+      hipError_t e = hipMalloc(&c->Vif, sizeof(double) * afn);
+      if (e == hipSuccess) e = hipMalloc(&c->Vf, sizeof(double) * afn);
+      arrange_fold_A(n, c->hVi, 1, c->Vif_e0, hf);
+      if (e == hipSuccess) e = hipMemcpy(c->Vif, hf, sizeof(double) * afn, hipMemcpyHostToDevice);
+      arrange_fold_A(n, c->hV, 0, c->Vf_e0, hf);
+      if (e == hipSuccess) e = hipMemcpy(c->Vf, hf, sizeof(double) * afn, hipMemcpyHostToDevice);
+      free(hf);
+      HCHK(c, e);
+    }
   } else {
     etd_fields<float> &F = c->f32;
     HCHK(c, hipMalloc(&F.u, sizeof(float) * n3 * 2 * V));  // [u | N1]
@@ -379,6 +392,8 @@ extern "C" void etd_close(etd_ctx *c) {
   (void)hipFree(c->gtmp);
   (void)hipFree(c->V4);
   (void)hipFree(c->Vi4);
+  (void)hipFree(c->Vf);
+  (void)hipFree(c->Vif);
   (void)hipFree(c->DDX);
   (void)hipFree(c->lam);
   (void)hipFree(c->Z);
@@ -588,6 +603,16 @@ void modeprod3(etd_ctx *c, int forward, const T *in, T *out, int nf, int accumul
   const etd_fields<T> F = fields<T>(c);
   if (c->prof) c->mp_fields += 3LL * nf;
   if constexpr (sizeof(T) == 8) {
+    // mp_variant 1: half the flop where the basis has parity; the other
+    // variants, and bases without it, take the full product
+    if (c->mp_variant == 1 && c->Vf) {
+      const double *A = forward ? c->Vif : c->Vf;
+      const int e0 = forward ? c->Vif_e0 : c->Vf_e0;
+      launch_modeprod_fold(c, A, forward, e0, in, n3, F.w1, n3, nf, 0);
+      launch_modeprod_fold(c, A, forward, e0, F.w1, n3, F.w2, n3, nf, 0);
+      launch_modeprod_fold(c, A, forward, e0, F.w2, n3, out, n3, nf, accumulate);
+      return;
+    }
     const double *A = forward ? c->Vi4 : c->V4;
     launch_modeprod(c, A, in, n3, F.w1, n3, nf, 1, 0);
     launch_modeprod(c, A, F.w1, n3, F.w2, n3, nf, 1, 0);
@@ -952,10 +977,17 @@ extern "C" int etd_k_modeprod(etd_ctx *c, int n, const double *A, const double *
     (void)hipFree(dout);
     return rc;
   }
+  // the step's rule: a matrix with parity is folded (columns' parity first)
+  int e0 = 0, fold = 0, fwd = 0;
+  if (rotate == 1 && c->mp_variant == 1) fold = (fwd = fold_parity(n, A, 1, &e0)) || fold_parity(n, A, 0, &e0);
   const int MT = (n + 15) / 16, nkc = (n + 15) / 16;
-  const size_t a4n = arrange_A_chunk(MT) * nkc;
+  const size_t a4n = fold ? fold_A_doubles(n) : arrange_A_chunk(MT) * nkc;
   double *h4 = (double *)malloc(sizeof(double) * a4n);
-  arrange_A(n, A, h4, MT, nkc);
+  if (!h4) return ETD_ERR_NOMEM;
+  if (fold)
+    arrange_fold_A(n, A, fwd, e0, h4);
+  else
+    arrange_A(n, A, h4, MT, nkc);
   double *dA, *din, *dout;
   HCHK(c, hipMalloc(&dA, sizeof(double) * a4n));
   HCHK(c, hipMalloc(&din, sizeof(double) * c->n3));
@@ -963,7 +995,10 @@ extern "C" int etd_k_modeprod(etd_ctx *c, int n, const double *A, const double *
   HCHK(c, hipMemcpy(dA, h4, sizeof(double) * a4n, hipMemcpyHostToDevice));
   HCHK(c, hipMemcpy(din, in, sizeof(double) * c->n3, hipMemcpyHostToDevice));
   free(h4);
-  launch_modeprod(c, dA, din, c->n3, dout, c->n3, 1, rotate, 0);
+  if (fold)
+    launch_modeprod_fold(c, dA, fwd, e0, din, c->n3, dout, c->n3, 1, 0);
+  else
+    launch_modeprod(c, dA, din, c->n3, dout, c->n3, 1, rotate, 0);
   HCHK(c, hipGetLastError());
   HCHK(c, hipStreamSynchronize(c->stream));
   HCHK(c, hipMemcpy(out, dout, sizeof(double) * c->n3, hipMemcpyDeviceToHost));

@@ -69,6 +69,10 @@ struct etd_ctx {
   /* device */
   double *u, *N1, *N2, *w1, *w2, *spec;
   double *V4, *Vi4;        /* MFMA-arranged A operands */
+  /* the same for the folded products (etd_fold.hip), where V and V^-1 have
+   * the parity they need (null otherwise); *_e0: the index of the first even mode */
+  double *Vf, *Vif;
+  int Vf_e0, Vif_e0;
   double *DDX, *DDY, *DDZ; /* D / h^2 per axis */
   double *lam;             /* nac x 9 */
   double *gtmp;            /* 3 x n3 gradient scratch for F2, or CH t */
@@ -151,7 +155,8 @@ struct etd_ctx {
   double *hpart;           /* pinned host copy */
   int npart;
   /* profiling */
-  int mp_variant;          /* 0..2: direct-to-LDS 4x4x4 (1 is the default), 4: register-staged 4x4x4, 16: 16x16x4 */
+  int mp_variant;          /* 0..2: direct-to-LDS 4x4x4 (1 is the default, and folds a basis with parity),
+                              4: register-staged 4x4x4, 16: 16x16x4 */
   int mp_nb;               /* column groups per wave of the 4x4x4 kernel (4 or 8) */
   int prof;                /* record per-class event pairs */
   hipEvent_t *ev;
@@ -336,6 +341,13 @@ void stage_forward(etd_ctx *c);
 template <typename T>
 int step_once_t(etd_ctx *c);
 
+/* folded products (etd_fold.hip): out = A in over the fastest axis, rotated,
+ * for A with parity (fold_parity) arranged by arrange_fold_A */
+int fold_parity(int n, const double *A, int forward, int *first);
+size_t fold_A_doubles(int n);
+void arrange_fold_A(int n, const double *A, int forward, int e0, double *Af);
+void launch_modeprod_fold(etd_ctx *c, const double *Af, int forward, int e0, const double *in, size_t in_fs,
+                          double *out, size_t out_fs, int nfields, int accumulate);
 void launch_modeprod(etd_ctx *c, const double *A4, const double *in, size_t in_fs, double *out, size_t out_fs,
                      int nfields, int rotate, int accumulate);
 void launch_copy16(etd_ctx *c, const void *in, void *out, size_t n16);
