@@ -127,6 +127,28 @@ static int validate(etd_ctx *c, const etd_params *p) {
   return ETD_OK;
 }
 
+// the full-size arrangement of V and V^-1, made when the context's mode
+// products need it (mp_variant other than 1, or a basis without parity)
+int full_basis(etd_ctx *c) {
+  if (c->mixed || c->V4 || (c->mp_variant == 1 && c->Vf)) return ETD_OK;
+  const int n = c->n, MT = (n + 15) / 16, nkc = (n + 15) / 16;
+  const size_t a4n = arrange_A_chunk(MT) * nkc;
+  double *h4 = (double *)malloc(sizeof(double) * 2 * a4n), *d = nullptr;
+  if (!h4) return seterr(c, ETD_ERR_NOMEM, "basis");
+  arrange_A(n, c->hVi, h4, MT, nkc);
+  arrange_A(n, c->hV, h4 + a4n, MT, nkc);
+  hipError_t e = hipMalloc(&d, sizeof(double) * 2 * a4n);
+  if (e == hipSuccess) e = hipMemcpy(d, h4, sizeof(double) * 2 * a4n, hipMemcpyHostToDevice);
+  free(h4);
+  if (e != hipSuccess) {
+    (void)hipFree(d);
+    HCHK(c, e);
+  }
+  c->Vi4 = d;
+  c->V4 = d + a4n;
+  return ETD_OK;
+}
+
 extern "C" int etd_create(const etd_params *p, const double *Vh, const double *Vih, const double *Dh, etd_ctx **out) {
   if (!p || !out) return ETD_ERR_ARG;
   *out = nullptr;
@@ -157,6 +179,7 @@ extern "C" int etd_create(const etd_params *p, const double *Vh, const double *V
   c->Ne = c->px * c->N;  // px = py = pz whenever elastic; the grid edge only matters then
   c->Ne3 = (size_t)c->Ne * c->Ne * c->Ne;
   *out = c;  // from here on etd_close releases partial state
+  host_copy_open();
   c->hV = (double *)malloc(sizeof(double) * n * n);
   c->hVi = (double *)malloc(sizeof(double) * n * n);
   c->hD = (double *)malloc(sizeof(double) * n);
@@ -221,30 +244,21 @@ extern "C" int etd_create(const etd_params *p, const double *Vh, const double *V
     c->bN2 = c->N2;
     c->bspec = c->spec;
     HCHK(c, hipMalloc(&c->gtmp, sizeof(double) * n3 * 3));
-    // eigenbasis as MFMA A fragments
-    const int MT = (n + 15) / 16, nkc = (n + 15) / 16;
-    const size_t a4n = arrange_A_chunk(MT) * nkc;
-    double *h4 = (double *)malloc(sizeof(double) * a4n);
-    HCHK(c, hipMalloc(&c->V4, sizeof(double) * a4n));
-    HCHK(c, hipMalloc(&c->Vi4, sizeof(double) * a4n));
-    arrange_A(n, c->hVi, h4, MT, nkc);
-    HCHK(c, hipMemcpy(c->Vi4, h4, sizeof(double) * a4n, hipMemcpyHostToDevice));
-    arrange_A(n, c->hV, h4, MT, nkc);
-    HCHK(c, hipMemcpy(c->V4, h4, sizeof(double) * a4n, hipMemcpyHostToDevice));
-    free(h4);
+    // eigenbasis as MFMA A fragments: folded, or (no parity, or another
+    // variant asked for) full-size
     if (fold_parity(n, c->hVi, 1, &c->Vif_e0) && fold_parity(n, c->hV, 0, &c->Vf_e0)) {
       const size_t afn = fold_A_doubles(n);
-      double *hf = (double *)malloc(sizeof(double) * afn);
+      double *hf = (double *)malloc(sizeof(double) * 2 * afn);
       if (!hf) return seterr(c, ETD_ERR_NOMEM, "folded basis");
-      hipError_t e = hipMalloc(&c->Vif, sizeof(double) * afn);
-      if (e == hipSuccess) e = hipMalloc(&c->Vf, sizeof(double) * afn);
       arrange_fold_A(n, c->hVi, 1, c->Vif_e0, hf);
-      if (e == hipSuccess) e = hipMemcpy(c->Vif, hf, sizeof(double) * afn, hipMemcpyHostToDevice);
-      arrange_fold_A(n, c->hV, 0, c->Vf_e0, hf);
-      if (e == hipSuccess) e = hipMemcpy(c->Vf, hf, sizeof(double) * afn, hipMemcpyHostToDevice);
+      arrange_fold_A(n, c->hV, 0, c->Vf_e0, hf + afn);
+      hipError_t e = hipMalloc(&c->Vif, sizeof(double) * 2 * afn);
+      if (e == hipSuccess) e = hipMemcpy(c->Vif, hf, sizeof(double) * 2 * afn, hipMemcpyHostToDevice);
       free(hf);
       HCHK(c, e);
+      c->Vf = c->Vif + afn;
     }
+    if ((rc = full_basis(c))) return rc;
   } else {
     etd_fields<float> &F = c->f32;
     HCHK(c, hipMalloc(&F.u, sizeof(float) * n3 * 2 * V));  // [u | N1]
@@ -390,9 +404,7 @@ extern "C" void etd_close(etd_ctx *c) {
   (void)hipFree(c->w2);
   (void)hipFree(c->spec);
   (void)hipFree(c->gtmp);
-  (void)hipFree(c->V4);
   (void)hipFree(c->Vi4);
-  (void)hipFree(c->Vf);
   (void)hipFree(c->Vif);
   (void)hipFree(c->DDX);
   (void)hipFree(c->lam);
@@ -416,6 +428,7 @@ extern "C" void etd_close(etd_ctx *c) {
   (void)hipFree(c->f32.E);
   (void)hipFree(c->V3);
   (void)hipFree(c->Vi3);
+  host_copy_close(c);
   for (int i = 0; i < c->cap_ev; i++) (void)hipEventDestroy(c->ev[i]);
   free(c->ev);
   free(c->ev_class);
@@ -476,26 +489,16 @@ extern "C" int etd_open(const char *dir, const char *suffix, etd_ctx **out) {
 }
 
 // ------------------------------------------------------------------ fields
-// host FP64 <-> device FP32 through a temporary host buffer (mixed path)
+static int copied(etd_ctx *c, hipError_t e) {
+  if (e == hipErrorOutOfMemory) return ETD_ERR_NOMEM;
+  return e == hipSuccess ? ETD_OK : seterr(c, ETD_ERR_DEVICE, "host copy: %s", hipGetErrorString(e));
+}
+// host FP64 <-> device FP32 (mixed path)
 static int put_f32(etd_ctx *c, float *dev, const double *host, size_t cnt) {
-  float *t = (float *)malloc(sizeof(float) * cnt);
-  if (!t) return ETD_ERR_NOMEM;
-  for (size_t i = 0; i < cnt; i++) t[i] = (float)host[i];
-  hipError_t e = hipMemcpy(dev, t, sizeof(float) * cnt, hipMemcpyHostToDevice);
-  free(t);
-  if (e != hipSuccess) return seterr(c, ETD_ERR_DEVICE, "hipMemcpy: %s", hipGetErrorString(e));
-  return ETD_OK;
+  return copied(c, host_copy<float>(c, dev, (double *)host, cnt, 1));
 }
 static int get_f32(etd_ctx *c, double *host, const float *dev, size_t cnt) {
-  float *t = (float *)malloc(sizeof(float) * cnt);
-  if (!t) return ETD_ERR_NOMEM;
-  hipError_t e = hipStreamSynchronize(c->stream);
-  if (e == hipSuccess) e = hipMemcpy(t, dev, sizeof(float) * cnt, hipMemcpyDeviceToHost);
-  if (e == hipSuccess)
-    for (size_t i = 0; i < cnt; i++) host[i] = t[i];
-  free(t);
-  if (e != hipSuccess) return seterr(c, ETD_ERR_DEVICE, "hipMemcpy: %s", hipGetErrorString(e));
-  return ETD_OK;
+  return copied(c, host_copy<float>(c, (float *)dev, host, cnt, 0));
 }
 
 extern "C" int etd_set_field(etd_ctx *c, int var, const double *host) {
@@ -505,9 +508,7 @@ extern "C" int etd_set_field(etd_ctx *c, int var, const double *host) {
   c->ch_stale = 1;
   if (c->mixed) return put_f32(c, c->f32.u + c->n3 * var, host, c->n3);
   for (int b = 0; b < c->P; b++)  // a decomposed run: the boxes one after another
-    HCHK(c, hipMemcpyAsync(c->bu + b * c->bs + c->n3 * var, host + b * c->n3, sizeof(double) * c->n3,
-                           hipMemcpyHostToDevice, c->stream));
-  HCHK(c, hipStreamSynchronize(c->stream));
+    HCHK(c, host_copy<double>(c, c->bu + b * c->bs + c->n3 * var, (double *)host + b * c->n3, c->n3, 1));
   return ETD_OK;
 }
 
@@ -537,9 +538,7 @@ extern "C" int etd_get_field(etd_ctx *c, int var, double *host) {
   if (!c || !host || var < 0 || var >= c->V) return seterr(c, ETD_ERR_ARG, "get_field: bad variable %d", var);
   if (c->mixed) return get_f32(c, host, c->f32.u + c->n3 * var, c->n3);
   for (int b = 0; b < c->P; b++)
-    HCHK(c, hipMemcpyAsync(host + b * c->n3, c->bu + b * c->bs + c->n3 * var, sizeof(double) * c->n3,
-                           hipMemcpyDeviceToHost, c->stream));
-  HCHK(c, hipStreamSynchronize(c->stream));
+    HCHK(c, host_copy<double>(c, c->bu + b * c->bs + c->n3 * var, host + b * c->n3, c->n3, 0));
   return ETD_OK;
 }
 

@@ -164,7 +164,12 @@ extern "C" int etd_set_tuning(etd_ctx *c, const etd_tuning *t) {
   if (!(v == 0 || v == 1 || v == 2 || v == 4 || v == 16)) return ETD_ERR_ARG;
   if (!(t->split_waves == 0 || t->split_waves == 4 || t->split_waves == 8)) return ETD_ERR_ARG;
   if (!(t->fft_variant == 0 || t->fft_variant == 1)) return ETD_ERR_ARG;
+  const int old = c->mp_variant;
   c->mp_variant = v;
+  if (int rc = full_basis(c)) {
+    c->mp_variant = old;
+    return rc;
+  }
   c->split_waves = t->split_waves;
   c->fft_variant = t->fft_variant;
   return ETD_OK;

@@ -34,8 +34,12 @@
 // bound is what rounding leaves of the symmetry in a computed basis (angles
 // up to 2 pi, an inversion: 6 eps for id 3, 67 eps for id 0 up to n = 272);
 // bases read from files are symmetric to 1e-12 only and keep the full product.
+// Even edges up to 32 keep the full product too: a launch is all it costs
+// there (4 and 8 fields: 2.9 us full, 2.8 to 3.0 us folded at n = 12, 3.8
+// against 3.2 to 3.4 us at n = 20; from n = 36 on 5.6 against 4.7 us and
+// more).  The full product of an odd edge is the slow one at any size.
 int fold_parity(int n, const double *A, int forward, int *first) {
-  if (n < 8) return 0;
+  if (n < 8 || (n % 2 == 0 && n <= 32)) return 0;
   double big = 0.0;
   for (size_t l = 0; l < (size_t)n * n; l++) {
     if (!(fabs(A[l]) <= DBL_MAX)) return 0;

@@ -1,0 +1,288 @@
+// etd_hostcopy.hip -- fields between the host's pageable memory (FP64) and
+// the device (FP64 or FP32).
+//
+// A copy to or from pageable memory goes through the runtime's pinned buffer
+// on one thread: 17 GB/s for the 60 MB of an FP64 field at n = 196, and for
+// FP32 storage a second pass on that thread converts, into pages that are
+// fresh each time.  Here a field passes through three pinned slots: the calling thread keeps the copies going, up to HC_THREADS
+// others convert (or copy) their share of each chunk that has arrived.
+// Measured, one field read (set), before against now: n = 196 FP64 3.4 (2.0)
+// -> 1.4 (1.4) ms, FP32 3.5 (2.7) -> 0.8 (0.8) ms; n = 260 FP32 21.8 (16.3)
+// -> 1.6 (1.7) ms; n = 36 FP32 88 -> 41 us.  Chunks: a copy costs about 13 us
+// besides its bytes, so 512 KiB pieces reach 21 GB/s, 4 MiB 43 GB/s; more
+// than 4 threads add nothing.
+#include <hip/hip_runtime.h>
+#include <emmintrin.h>
+#include <pthread.h>
+#include <stdlib.h>
+#include <string.h>
+
+#include <atomic>
+#include <mutex>
+#include <utility>
+
+#include "etd_internal.h"
+
+#define HC_THREADS 4
+#define HC_CHUNK ((size_t)4 << 20)   // most device bytes per slot
+#define HC_SHARE ((size_t)8 << 20)   // host bytes that pay for one more thread (from two on)
+#define HC_SLOTS 3
+#define HC_MIN ((size_t)64 << 10)    // least device bytes per slot
+#define HC_DIRECT ((size_t)1 << 20)  // FP64 up to this: the runtime's own path
+
+// host FP64 values from device ones, past the cache for long runs
+static void widen(double *dst, const double *src, size_t cnt) { memcpy(dst, src, sizeof(double) * cnt); }
+static void widen(double *dst, const float *src, size_t cnt) {
+  size_t i = 0;
+  if (cnt >= 32768 && ((uintptr_t)dst & 7) == 0) {
+    if ((uintptr_t)dst & 15) {
+      dst[0] = src[0];
+      i = 1;
+    }
+    for (; i + 4 <= cnt; i += 4) {
+      const __m128 v = _mm_loadu_ps(src + i);
+      _mm_stream_pd(dst + i, _mm_cvtps_pd(v));
+      _mm_stream_pd(dst + i + 2, _mm_cvtps_pd(_mm_movehl_ps(v, v)));
+    }
+    _mm_sfence();
+  }
+  for (; i < cnt; i++) dst[i] = src[i];
+}
+static void narrow(double *dst, const double *src, size_t cnt) { memcpy(dst, src, sizeof(double) * cnt); }
+static void narrow(float *dst, const double *src, size_t cnt) {
+  for (size_t i = 0; i < cnt; i++) dst[i] = (float)src[i];
+}
+
+template <typename T>
+struct hc_job {
+  etd_ctx *c;
+  T *dev;
+  double *host;
+  size_t cnt, per;  // elements in all, per chunk
+  size_t nch;       // chunks
+  int put;
+  // the workers' side: chunks they may take, chunks each has finished
+  int nt;
+  std::atomic<size_t> ready;
+  std::atomic<size_t> done[HC_THREADS];
+  std::atomic<int> stop;
+
+  void *pin;        // HC_SLOTS chunks
+
+  T *slot(size_t k) const { return (T *)pin + (k % HC_SLOTS) * per; }
+  size_t len(size_t k) const { return (k + 1) * per <= cnt ? per : cnt - k * per; }
+  // elements [a, b) of chunk k between its slot and the host
+  void part(size_t k, size_t a, size_t b) const {
+    if (put) narrow(slot(k) + a, host + k * per + a, b - a);
+    else widen(host + k * per + a, slot(k) + a, b - a);
+  }
+  hipError_t start(size_t k) const {
+    const size_t b = sizeof(T) * len(k);
+    hipError_t e = put ? hipMemcpyAsync(dev + k * per, slot(k), b, hipMemcpyHostToDevice, c->stream)
+                       : hipMemcpyAsync(slot(k), dev + k * per, b, hipMemcpyDeviceToHost, c->stream);
+    return e != hipSuccess ? e : hipEventRecord(c->io_ev[k % HC_SLOTS], c->stream);
+  }
+  hipError_t wait(size_t k) const { return hipEventSynchronize(c->io_ev[k % HC_SLOTS]); }
+};
+
+template <typename T>
+struct hc_arg {
+  hc_job<T> *j;
+  int t;
+};
+
+// a worker converts (or copies) its share of every chunk; it makes no HIP
+// call (a thread's first one costs a few hundred microseconds)
+template <typename T>
+static void *hc_thread(void *p) {
+  hc_job<T> *j = ((hc_arg<T> *)p)->j;
+  const int t = ((hc_arg<T> *)p)->t;
+  for (size_t k = 0; k < j->nch; k++) {
+    while (j->ready.load(std::memory_order_acquire) <= k) {
+      if (j->stop.load(std::memory_order_relaxed)) return nullptr;
+      _mm_pause();
+    }
+    // shares in whole cache lines of the host buffer
+    const size_t n = j->len(k), nt = j->nt, sh = ((n + nt - 1) / nt + 7) & ~(size_t)7;
+    const size_t a = t * sh < n ? t * sh : n, b = a + sh < n ? a + sh : n;
+    if (b > a) j->part(k, a, b);
+    j->done[t].store(k + 1, std::memory_order_release);
+  }
+  return nullptr;
+}
+
+// the calling thread: copies and events, and the conversion itself when
+// there are no workers
+template <typename T>
+static hipError_t hc_run(hc_job<T> *j) {
+  hipError_t e = hipSuccess;
+  auto finish = [&](size_t k) {  // the host side of chunk k
+    if (j->nt == 0) return j->part(k, 0, j->len(k));
+    j->ready.store(k + 1, std::memory_order_release);
+  };
+  auto finished = [&](size_t k) {
+    for (int t = 0; t < j->nt; t++)
+      while (j->done[t].load(std::memory_order_acquire) <= k) _mm_pause();
+  };
+  if (j->put) {
+    for (size_t k = 0; k <= j->nch; k++) {
+      if (k < j->nch) {
+        if (k >= HC_SLOTS && (e = j->wait(k - HC_SLOTS)) != hipSuccess) return e;
+        finish(k);
+      }
+      if (k == 0) continue;
+      finished(k - 1);
+      if ((e = j->start(k - 1)) != hipSuccess) return e;
+    }
+    return e;
+  }
+  for (size_t k = 0; k < j->nch && k < HC_SLOTS; k++)
+    if ((e = j->start(k)) != hipSuccess) return e;
+  for (size_t k = 0; k < j->nch; k++) {
+    if ((e = j->wait(k)) != hipSuccess) return e;
+    finish(k);
+    if (k == 0 || k - 1 + HC_SLOTS >= j->nch) continue;
+    finished(k - 1);
+    if ((e = j->start(k - 1 + HC_SLOTS)) != hipSuccess) return e;
+  }
+  if (j->nch) finished(j->nch - 1);
+  return e;
+}
+
+// Pinned memory for a call's slots.  It is taken for the call and given back
+// after it (a copy is over when it returns), so contexts share it: allocating
+// it per context cost an ensemble of 20 a millisecond each.  At most
+// HC_POOL buffers wait between calls; the last context to close frees them.
+#define HC_POOL 4
+static std::mutex pool_mu;
+static struct {
+  void *p;
+  size_t bytes;
+} pool_buf[HC_POOL];
+static int pool_n, pool_users;
+
+static void *pool_take(size_t need, size_t *bytes) {
+  {
+    std::lock_guard<std::mutex> l(pool_mu);
+    for (int i = 0; i < pool_n; i++)
+      if (pool_buf[i].bytes >= need) {
+        void *p = pool_buf[i].p;
+        *bytes = pool_buf[i].bytes;
+        pool_buf[i] = pool_buf[--pool_n];
+        return p;
+      }
+  }
+  void *p = nullptr;
+  if (hipHostMalloc(&p, need, hipHostMallocPortable) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  *bytes = need;
+  return p;
+}
+static void pool_give(void *p, size_t bytes) {
+  if (!p) return;
+  {
+    std::lock_guard<std::mutex> l(pool_mu);
+    if (pool_users > 0) {
+      if (pool_n < HC_POOL) {
+        pool_buf[pool_n++] = {p, bytes};
+        return;
+      }
+      for (int i = 0; i < pool_n; i++)  // full: the larger one stays
+        if (pool_buf[i].bytes < bytes) {
+          std::swap(pool_buf[i].p, p);
+          std::swap(pool_buf[i].bytes, bytes);
+        }
+    }
+  }
+  (void)hipHostFree(p);
+}
+void host_copy_open(void) {
+  std::lock_guard<std::mutex> l(pool_mu);
+  pool_users++;
+}
+void host_copy_close(etd_ctx *c) {
+  for (int i = 0; i < c->io_nev; i++) (void)hipEventDestroy(c->io_ev[i]);
+  std::lock_guard<std::mutex> l(pool_mu);
+  if (--pool_users == 0)
+    while (pool_n) (void)hipHostFree(pool_buf[--pool_n].p);
+}
+
+// the slots' events; 0 when they cannot be had
+static int hc_events(etd_ctx *c) {
+  for (; c->io_nev < HC_SLOTS; c->io_nev++)
+    if (hipEventCreateWithFlags(&c->io_ev[c->io_nev], hipEventDisableTiming) != hipSuccess) {
+      (void)hipGetLastError();
+      return 0;
+    }
+  return 1;
+}
+
+// the copy without slots of its own: FP64 directly, FP32 through a temporary
+static hipError_t hc_plain(etd_ctx *c, double *dev, double *host, size_t cnt, int put) {
+  hipError_t e = put ? hipMemcpyAsync(dev, host, sizeof(double) * cnt, hipMemcpyHostToDevice, c->stream)
+                     : hipMemcpyAsync(host, dev, sizeof(double) * cnt, hipMemcpyDeviceToHost, c->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  return e;
+}
+static hipError_t hc_plain(etd_ctx *c, float *dev, double *host, size_t cnt, int put) {
+  float *t = (float *)malloc(sizeof(float) * cnt);
+  if (!t) return hipErrorOutOfMemory;
+  hipError_t e = hipSuccess;
+  if (put) {
+    narrow(t, host, cnt);
+    e = hipMemcpyAsync(dev, t, sizeof(float) * cnt, hipMemcpyHostToDevice, c->stream);
+  } else {
+    e = hipMemcpyAsync(t, dev, sizeof(float) * cnt, hipMemcpyDeviceToHost, c->stream);
+  }
+  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  if (e == hipSuccess && !put) widen(host, t, cnt);
+  free(t);
+  return e;
+}
+
+template <typename T>
+hipError_t host_copy(etd_ctx *c, T *dev, double *host, size_t cnt, int put) {
+  const size_t bytes = sizeof(T) * cnt;
+  if (sizeof(T) == 8 && bytes <= HC_DIRECT) return hc_plain(c, dev, host, cnt, put);
+  // a quarter of the field per chunk, at most HC_CHUNK, in whole 4 KiB; half
+  // of it up to 4 MiB (quarters that short took 430 us from the device at
+  // 1 MiB, halves 70 us)
+  size_t per = (bytes / (bytes <= HC_CHUNK ? 2 : 4) + 4095) / 4096 * 4096;
+  per = per < HC_MIN ? HC_MIN : per > HC_CHUNK ? HC_CHUNK : per;
+  const size_t nch = (bytes + per - 1) / per;
+  size_t pinned = 0;
+  void *pin = hc_events(c) ? pool_take((nch < HC_SLOTS ? nch : HC_SLOTS) * per, &pinned) : nullptr;
+  if (!pin) return hc_plain(c, dev, host, cnt, put);
+  hc_job<T> job;
+  job.pin = pin;
+  job.c = c;
+  job.dev = dev;
+  job.host = host;
+  job.cnt = cnt;
+  job.per = per / sizeof(T);
+  job.nch = nch;
+  job.put = put;
+  job.ready = 0;
+  job.stop = 0;
+  hc_arg<T> arg[HC_THREADS];
+  pthread_t th[HC_THREADS];
+  int want = (int)(sizeof(double) * cnt / HC_SHARE), made = 0;
+  want = want < 2 ? 0 : want > HC_THREADS ? HC_THREADS : want;
+  for (; made < want; made++) {
+    job.done[made] = 0;
+    arg[made] = hc_arg<T>{&job, made};
+    if (pthread_create(&th[made], nullptr, hc_thread<T>, &arg[made])) break;  // fewer threads, or none, do as well
+  }
+  job.nt = made;  // read by a worker after its first chunk is ready
+  hipError_t e = hc_run(&job);
+  job.stop = 1;
+  for (int t = 0; t < made; t++) (void)pthread_join(th[t], nullptr);
+  // the slots are free, and what was put is on the device, after this
+  const hipError_t es = hipStreamSynchronize(c->stream);
+  pool_give(pin, pinned);
+  return e != hipSuccess ? e : es;
+}
+template hipError_t host_copy<double>(etd_ctx *, double *, double *, size_t, int);
+template hipError_t host_copy<float>(etd_ctx *, float *, double *, size_t, int);

@@ -68,9 +68,10 @@ struct etd_ctx {
   double *hV, *hVi, *hD;
   /* device */
   double *u, *N1, *N2, *w1, *w2, *spec;
-  double *V4, *Vi4;        /* MFMA-arranged A operands */
-  /* the same for the folded products (etd_fold.hip), where V and V^-1 have
-   * the parity they need (null otherwise); *_e0: the index of the first even mode */
+  double *V4, *Vi4;        /* MFMA-arranged A operands, one allocation from Vi4 (null until needed) */
+  /* the same for the folded products (etd_fold.hip), one allocation from Vif,
+   * where V and V^-1 have the parity they need (null otherwise); *_e0: the
+   * index of the first even mode */
   double *Vf, *Vif;
   int Vf_e0, Vif_e0;
   double *DDX, *DDY, *DDZ; /* D / h^2 per axis */
@@ -150,6 +151,9 @@ struct etd_ctx {
   int blas_status;         /* first failing rocBLAS status of the correction since the last check */
   long long mp_fields;     /* field passes of the mode-product launches while timing */
   long long ad_fetches;    /* host fetches of the adaptive partial sums */
+  /* events of the host copies' pinned slots (etd_hostcopy.hip), made on first use */
+  hipEvent_t io_ev[3];
+  int io_nev;
   /* energy partials */
   double *part;            /* device partial sums */
   double *hpart;           /* pinned host copy */
@@ -341,6 +345,14 @@ void stage_forward(etd_ctx *c);
 template <typename T>
 int step_once_t(etd_ctx *c);
 
+int full_basis(etd_ctx *c);
+/* cnt values between host FP64 (pageable) and the device, put: to the device;
+ * returns when the host buffer is free (put) or filled */
+template <typename T>
+hipError_t host_copy(etd_ctx *c, T *dev, double *host, size_t cnt, int put);
+/* every context opens and closes once: the copies' pinned memory is shared */
+void host_copy_open(void);
+void host_copy_close(etd_ctx *c);
 /* folded products (etd_fold.hip): out = A in over the fastest axis, rotated,
  * for A with parity (fold_parity) arranged by arrange_fold_A */
 int fold_parity(int n, const double *A, int forward, int *first);
