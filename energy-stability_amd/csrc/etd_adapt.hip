@@ -136,13 +136,27 @@ __device__ inline void block_sum2(double a, double b, double *__restrict__ part)
 template <typename T>
 __global__ __launch_bounds__(256) void k_elastic_energy(const T *__restrict__ u, const T *__restrict__ E, int n, int g,
                                                         int nac, int ring, int slot0,
-                                                        double *__restrict__ part) {
+                                                        const double *__restrict__ ev, double *__restrict__ part) {
   const int N = n - 2 * g;
   const size_t N3 = (size_t)N * N * N, n3 = (size_t)n * n * n;
   double acc = 0.0, aabs = 0.0;
   FOR_INTERIOR_CELLS(N, x, y, z) {
     const size_t l = (((size_t)(z + g)) * n + (y + g)) * n + (x + g);
     const size_t m = ((size_t)z * N + y) * N + x;
+    if (ev) {  // el_mix: felas_p = ev_p . the six stress components
+      double sg[6];
+#pragma unroll
+      for (int c6 = 0; c6 < 6; c6++) sg[c6] = E[c6 * N3 + m];
+      for (int p = 0; p < nac; p++) {
+        double f = 0.0;
+#pragma unroll
+        for (int c6 = 0; c6 < 6; c6++) f += ev[6 * p + c6] * sg[c6];
+        const double t = (double)u[n3 * p + l] * f;
+        acc += t;
+        aabs += fabs(t);
+      }
+      continue;
+    }
     for (int p0 = 0; p0 < nac; p0 += FB) {
       T a[FB], b[FB];
 #pragma unroll
@@ -192,7 +206,7 @@ template <typename T>
 __global__ __launch_bounds__(256) void k_accept_stats(const T *__restrict__ u, const T *__restrict__ u0,
                                                       const T *__restrict__ E, const double *__restrict__ lam,
                                                       scheme_args a, int with_el, int ring, int slot0,
-                                                      double *__restrict__ part) {
+                                                      const double *__restrict__ ev, double *__restrict__ part) {
   const int n = a.n, g = a.g, N = n - 2 * g;
   const size_t N3 = (size_t)N * N * N, n3 = (size_t)n * n * n;
   const int V = a.nac + a.nch;
@@ -201,6 +215,10 @@ __global__ __launch_bounds__(256) void k_accept_stats(const T *__restrict__ u, c
     const cell_nb c = neighbours(n, g, N, x, y, z);
     const size_t m = ((size_t)z * N + y) * N + x;
     double s2 = 0.0, s3 = 0.0, e = 0.0, ea = 0.0, cell = 0.0;
+    T sg[6];  // el_mix: felas_p = ev_p . the six stress components
+    if (with_el && ev)
+#pragma unroll
+      for (int c6 = 0; c6 < 6; c6++) sg[c6] = E[c6 * N3 + m];
     for (int p0 = 0; p0 < V; p0 += FB) {
       T v[FB], v0[FB], vxp[FB], vyp[FB], vzp[FB], vxm[FB], vym[FB], vzm[FB], fe[FB];
 #pragma unroll
@@ -216,7 +234,7 @@ __global__ __launch_bounds__(256) void k_accept_stats(const T *__restrict__ u, c
         vzm[q] = f[c.zm];
         const int pa = p < a.nac ? p : 0;  // AC-only reads stay inside the AC fields
         v0[q] = u0[n3 * pa + c.l];
-        if (with_el) {
+        if (with_el && !ev) {
           int slot = slot0 + pa;  // pa < nac < ring
           if (slot >= ring) slot -= ring;
           fe[q] = E[(size_t)slot * N3 + m];
@@ -250,7 +268,14 @@ __global__ __launch_bounds__(256) void k_accept_stats(const T *__restrict__ u, c
           cell = fmax(cell, fabs(vv));
           gsum += (double)sqrtf((float)(gxc * gxc + gyc * gyc + gzc * gzc));
           if (with_el) {
-            const double t = vv * (double)fe[q];
+            double f = 0.0;
+            if (ev) {
+#pragma unroll
+              for (int c6 = 0; c6 < 6; c6++) f += ev[6 * p + c6] * (double)sg[c6];
+            } else {
+              f = fe[q];
+            }
+            const double t = vv * f;
             el += t;
             elabs += fabs(t);
           }
@@ -392,7 +417,8 @@ static int energy_of(etd_ctx *c, int kind, int with_elastic, double *E, double *
       launch_elastic<T>(c);
       const long long Lbase = (c->elastic_evals - 1) * (long long)c->nac;
       k_elastic_energy<T><<<RBLOCKS, 256, 0, c->stream>>>(F.u, F.E, c->n, c->g, c->nac, c->ring,
-                                                          (int)(Lbase % c->ring), c->ad_part);
+                                                          (int)(Lbase % c->ring),
+                                                          c->el_mix ? c->dconst->ev : nullptr, c->ad_part);
       if ((rc = fetch_part(c, 2))) return rc;
       double s = 0.0;
       for (int i = 0; i < RBLOCKS; i++) s += c->ad_hpart[i * RCOLS];
@@ -423,7 +449,7 @@ static int energy_of(etd_ctx *c, int kind, int with_elastic, double *E, double *
       slot0 = (int)(((c->elastic_evals - 1) * (long long)c->nac) % c->ring);
     }
     k_accept_stats<T><<<RBLOCKS, 256, 0, c->stream>>>(F.u, u0, F.E, c->lam, a, el_on ? 1 : 0, c->ring, slot0,
-                                                      c->ad_part);
+                                                      c->el_mix ? c->dconst->ev : nullptr, c->ad_part);
     if ((rc = fetch_part(c, 8))) return rc;
     double s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     for (int i = 0; i < RBLOCKS; i++) {

@@ -308,18 +308,21 @@ extern "C" int etd_create(const etd_params *p, const double *Vh, const double *V
   if (c->nel > 0) {
     c->fft_npass = fft_plan_radices(c->Ne, c->fft_radix);
     if (c->fft_npass < 0) return seterr(c, ETD_ERR_UNSUPPORTED, "N = %d has prime factors other than 2, 3, 5", c->Ne);
-    c->npair = (c->nel + 1) / 2;
+    c->el_mix = p->elastic == 1 && c->nel > 6;
+    c->nft = c->el_mix ? 6 : c->nel;
+    c->npair = (c->nft + 1) / 2;
     c->ring = c->nel + 2;
+    const int nE = c->el_mix ? 12 : c->ring;  // fields of E
     if (!c->mixed) {
       HCHK(c, hipMalloc(&c->Z, sizeof(double) * 2 * c->Ne3 * c->npair));
       HCHK(c, hipMalloc(&c->Y, sizeof(double) * 2 * c->Ne3 * c->npair));
-      HCHK(c, hipMalloc(&c->E, sizeof(double) * c->Ne3 * c->ring));
-      HCHK(c, hipMemsetAsync(c->E, 0, sizeof(double) * c->Ne3 * c->ring, c->stream));
+      HCHK(c, hipMalloc(&c->E, sizeof(double) * c->Ne3 * nE));
+      HCHK(c, hipMemsetAsync(c->E, 0, sizeof(double) * c->Ne3 * nE, c->stream));
     } else {
       HCHK(c, hipMalloc(&c->f32.Z, sizeof(float) * 2 * c->N3 * c->npair));
       HCHK(c, hipMalloc(&c->f32.Y, sizeof(float) * 2 * c->N3 * c->npair));
-      HCHK(c, hipMalloc(&c->f32.E, sizeof(float) * c->N3 * c->ring));
-      HCHK(c, hipMemsetAsync(c->f32.E, 0, sizeof(float) * c->N3 * c->ring, c->stream));
+      HCHK(c, hipMalloc(&c->f32.E, sizeof(float) * c->N3 * nE));
+      HCHK(c, hipMemsetAsync(c->f32.E, 0, sizeof(float) * c->N3 * nE, c->stream));
     }
     double *tw = (double *)malloc(sizeof(double) * 2 * c->Ne);
     const double pi = 3.14159265358979323846;
@@ -332,8 +335,22 @@ extern "C" int etd_create(const etd_params *p, const double *Vh, const double *V
     free(tw);
     etd_dev_consts *k = (etd_dev_consts *)calloc(1, sizeof(etd_dev_consts));
     c4_from_voigt(p->C, k->C4);
-    for (int q = 0; q < c->nel; q++) {
-      const double *e = p->eps0 + 9 * q;
+    // the transformed fields' eigenstrains: the variants', or the six unit
+    // strains and every variant's components of them
+    const double *eps = p->eps0;
+    double unit[6 * 9] = {0};
+    if (c->el_mix) {
+      static const int ij[6][2] = {{0, 0}, {1, 1}, {2, 2}, {1, 2}, {0, 2}, {0, 1}};
+      for (int a = 0; a < 6; a++) {
+        const int i = ij[a][0], j = ij[a][1];
+        unit[9 * a + 3 * i + j] = unit[9 * a + 3 * j + i] = 1.0;
+        for (int q = 0; q < c->nel; q++)
+          k->ev[6 * q + a] = i == j ? eps[9 * q + 4 * i] : 0.5 * (eps[9 * q + 3 * i + j] + eps[9 * q + 3 * j + i]);
+      }
+      eps = unit;
+    }
+    for (int q = 0; q < c->nft; q++) {
+      const double *e = eps + 9 * q;
       for (int i = 0; i < 3; i++)
         for (int j = 0; j < 3; j++) {
           double s = 0.0;
@@ -342,10 +359,10 @@ extern "C" int etd_create(const etd_params *p, const double *Vh, const double *V
           k->sig[9 * q + i * 3 + j] = s;
         }
     }
-    for (int a = 0; a < c->nel; a++)
-      for (int b = 0; b < c->nel; b++) {
+    for (int a = 0; a < c->nft; a++)
+      for (int b = 0; b < c->nft; b++) {
         double t0 = 0.0;
-        const double *ea = p->eps0 + 9 * a, *eb = p->eps0 + 9 * b;
+        const double *ea = eps + 9 * a, *eb = eps + 9 * b;
         for (int i = 0; i < 3; i++)
           for (int j = 0; j < 3; j++)
             for (int kk = 0; kk < 3; kk++)

@@ -10,7 +10,9 @@
  *   spec  2V x n3  spectral u-hat / N-hat in the rotated x'y'z' layout
  *   Vi4,V4         V^-1 and V rearranged as MFMA A-fragments (see modeprod)
  *   Z,Y   P x N^3  complex pairs (eta_2r + i eta_2r+1) for the elastic FFTs
- *   E     R x N^3  ring of elastic driving forces (interior), R = nac + 2
+ *   E     R x N^3  ring of elastic driving forces (interior), R = nac + 2;
+ *         with el_mix 12 x N^3: the six stress components of the latest
+ *         evaluation, then the previous one's on the box edges
  */
 #ifndef ETD_INTERNAL_H
 #define ETD_INTERNAL_H
@@ -45,6 +47,10 @@ struct etd_dev_consts {
   double C4[81];
   double sig[ETD_MAX_VAR * 9];
   double t0[ETD_MAX_VAR * ETD_MAX_VAR];
+  /* with el_mix: the six components of every variant's eigenstrain (xx, yy,
+   * zz, yz, xz, xy of its symmetric part); sig and t0 are then those of the
+   * six unit strains */
+  double ev[ETD_MAX_VAR * 6];
 };
 
 struct etd_ctx {
@@ -86,6 +92,9 @@ struct etd_ctx {
   /* the fields the elastic force acts on: AC fields (ELASTIC = 1) or CH
    * fields (ELASTIC = 2), nel of them from field el_v0; nel = 0 without */
   int nel, el_v0;
+  /* el_mix: more than six variants are transformed as the six strain
+   * components they span (nft = 6 fields instead of nel), see launch_elastic */
+  int el_mix, nft;
   long long elastic_evals; /* completed elastic evaluations */
   int elastic_fresh;       /* the latest evaluation is of the current fields (adaptive energy test) */
   int fft_radix[16], fft_npass;

@@ -752,6 +752,7 @@ struct nl_args {
   int P, px, py, pz, bx, by, bz;
   long long bs;
   int bxo, byo, bzo;
+  const double *ev;  // el_mix: the variants' six strain components (E then holds stresses), or null
 };
 
 // -1 / 0 / +1: the extended coordinate e lies before, in or after the interior
@@ -790,6 +791,22 @@ __device__ __forceinline__ int gwrap(int e, int o, int g, int Ng) {
 // a ghost of f carry values of earlier variants: with d = number of ghost
 // coordinates, the value is the interior of variant p - max(0, d-1) at the
 // fully wrapped position (variants before 0 come from the previous call).
+// With el_mix, E holds the six stress components the force is a combination
+// of, felas_p = sum_a ev_pa E_a: of the latest evaluation, then of the one
+// before it on the cells that have two or three coordinates within g of the
+// box (the only ones that any lag reads).
+template <typename T>
+__device__ __forceinline__ double felas_mix(const T *E, const nl_args &a, int p, int lag, size_t off) {
+  const size_t N3 = (size_t)a.N * a.N * a.N;
+  const int q = p - lag;
+  const double *ev = a.ev + 6 * (q < 0 ? q + a.nac : q);
+  const T *e = E + off + (q < 0 ? 6 * N3 : 0);
+  double s = 0.0;
+#pragma unroll 1
+  for (int c = 0; c < 6; c++) s += ev[c] * (double)e[c * N3];
+  return s;
+}
+
 template <typename T>
 __device__ __forceinline__ double felas_at(const T *E, const nl_args &a, int p, int k, int j, int i) {
   if (a.phys && (k < a.g || k >= a.n - a.g || j < a.g || j >= a.n - a.g || i < a.g || i >= a.n - a.g))
@@ -803,6 +820,7 @@ __device__ __forceinline__ double felas_at(const T *E, const nl_args &a, int p, 
   if (slot >= a.ring) slot -= a.ring;
   if (slot < 0) slot += a.ring;
   const int wk = gwrap(k, a.bzo, g, N), wj = gwrap(j, a.byo, g, N), wi = gwrap(i, a.bxo, g, N);
+  if (a.ev) return felas_mix(E, a, p, lag, ((size_t)wk * N + wj) * N + wi);
   return E[(size_t)slot * N * N * N + ((size_t)wk * N + wj) * N + wi];
 }
 
@@ -922,6 +940,107 @@ __global__ __launch_bounds__(256) void k_nonlin_ac(const T *__restrict__ u, T *_
       out[n3 * (unsigned)p + lo] = (T)f;
     }
   }
+}
+
+// The same with el_mix: the force of every field comes from the six stress
+// components, read once, and the fields stay in registers between the sum of
+// squares and their own terms (FB >= nac).  Bound by instruction issue as
+// much as by HBM (in k_nonlin_ac's form it took 440 us at 196^3 x 12 FP32),
+// so every access is one base plus one 32-bit byte offset, and what only
+// cells near the faces need is skipped by waves that have none: 238 us, 372
+// us in FP64 (3.8 and 4.9 TB/s of the 30 field passes).  Reading the lagged
+// cells' values field by field made the few waves that have them the longest.
+template <typename T, int FB>
+__global__ __launch_bounds__(256) void k_nonlin_mix(const T *__restrict__ u, T *__restrict__ out,
+                                                    const T *__restrict__ sub, const T *__restrict__ E, nl_args a,
+                                                    int mask_here, const double *__restrict__ evs) {
+  const int n = a.n, g = a.g;
+  const unsigned n3 = (unsigned)n * n * n;
+  const size_t l = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (l >= n3) return;
+  int i, j, k;
+  idx3(l, n, i, j, k);
+  const unsigned lo = (unsigned)l * (unsigned)sizeof(T);  // n <= 272: bytes of a field fit 32 bits
+  auto at = [&](const T *f, unsigned b) { return *(const T *)((const char *)f + b); };
+  const unsigned N3 = (unsigned)a.N * a.N * a.N;
+  const bool fel_zero = a.phys && (k < g || k >= n - g || j < g || j >= n - g || i < g || i >= n - g);
+  const felas_cell fc = felas_locate(a, k, j, i);
+  const unsigned fo = (unsigned)fc.off * (unsigned)sizeof(T);
+  T uv[FB], sv[6];
+#pragma unroll
+  for (int e = 0; e < FB; e++) uv[e] = at(u + (size_t)n3 * (e < a.nac ? e : a.nac - 1), lo);
+#pragma unroll
+  for (int c = 0; c < 6; c++) sv[c] = at(E + (size_t)N3 * c, fo);
+  double sg[6];
+#pragma unroll
+  for (int c = 0; c < 6; c++) sg[c] = fel_zero ? 0.0 : (double)sv[c];
+  // a lagged cell takes the force of one or two variants earlier: the last
+  // ones of the loop over the fields (h1, h2), before variant 0 those of the
+  // previous evaluation
+  const bool lagged = fc.lag && !fel_zero, any_lag = __any(lagged);
+  double h1 = 0.0, h2 = 0.0;
+  if (lagged) {
+#pragma unroll
+    for (int c = 0; c < 6; c++) {
+      const double v = at(E + (size_t)N3 * (6 + c), fo);
+      h1 += evs[6 * (a.nac - 1) + c] * v;
+      h2 += evs[6 * (a.nac - 2) + c] * v;
+    }
+  }
+  // outside coupling, as in k_nonlin_ac
+  const bool fx = !a.phys && (i == 0 || i == n - 1), fy = !a.phys && (j == 0 || j == n - 1),
+             fz = !a.phys && (k == 0 || k == n - 1);
+  const bool any_face = __any(fx || fy || fz);
+  long long ox = 0, oy = 0, oz = 0;
+  if (any_face) {
+    const int wk = wrap_e(k, n, g), wj = wrap_e(j, n, g), wi = wrap_e(i, n, g);
+    const int sk = box_shift(k, n, g), sj = box_shift(j, n, g), si = box_shift(i, n, g);
+    if (fx) ox = (long long)IDX(n, wk, wj, wrap_e(i == 0 ? -1 : n, n, g)) + box_off(a, i == 0 ? -1 : 1, sj, sk);
+    if (fy) oy = (long long)IDX(n, wk, wrap_e(j == 0 ? -1 : n, n, g), wi) + box_off(a, si, j == 0 ? -1 : 1, sk);
+    if (fz) oz = (long long)IDX(n, wrap_e(k == 0 ? -1 : n, n, g), wj, wi) + box_off(a, si, sj, k == 0 ? -1 : 1);
+  }
+  double s = 0.0;
+#pragma unroll
+  for (int e = 0; e < FB; e++)
+    if (e < a.nac) s = s + (double)uv[e] * (double)uv[e];
+  const double ce = a.LE * a.epn2, ces = a.LE * a.es;
+  auto field = [&](auto et) {
+    constexpr int p = decltype(et)::value;
+    if (p >= a.nac) return;
+    const double up = uv[p];
+    double fe = 0.0;
+#pragma unroll
+    for (int c = 0; c < 6; c++) fe += evs[6 * p + c] * sg[c];
+    if (any_lag) {
+      const double own = fe;
+      fe = !lagged ? own : fc.lag == 1 ? h1 : h2;
+      h2 = h1;
+      h1 = own;
+    }
+    double f = a.LE * a.KE * up;
+    if (a.fe == 1) {  // CALPHAD driving force, as in k_nonlin_ac
+      const double dp = 30.0 * up * up * (1 - up) * (1 - up);
+      const double dq = 4.0 * CAL_WMEGA * up * (1 - up) * (2 - up);
+      const double dfeta = -(a.gbcc * dp) + (a.ghcp * dp) + dq;
+      f -= a.LE * (dfeta / CAL_GNORMAL + 4.0 * CAL_ALPHA * (up * (s - up * up)));
+    } else {
+      const double fp = a.a2 * up - a.a3 * up * up + a.a4 * s * up;
+      f -= a.LE * fp;
+    }
+    if (any_face) {
+      const T *uf = u + (size_t)n3 * p;
+      if (fx) f += ce * (double)uf[ox] / a.hx / a.hx;
+      if (fy) f += ce * (double)uf[oy] / a.hy / a.hy;
+      if (fz) f += ce * (double)uf[oz] / a.hz / a.hz;
+    }
+    f -= ces * fe;
+    if (mask_here && a.mask && a.mask[l] == 0) f -= 0.5 * up;
+    if (sub) f -= (double)at(sub + (size_t)n3 * p, lo);
+    *(T *)((char *)(out + (size_t)n3 * p) + lo) = (T)f;
+  };
+  [&]<size_t... I>(std::index_sequence<I...>) {
+    (field(std::integral_constant<int, (int)I>{}), ...);
+  }(std::make_index_sequence<FB>{});
 }
 
 // ac_calc_F2 (anisotropic.c:164-627), pass 1: G = Lambda (gx, gy, gz) with
@@ -1248,6 +1367,7 @@ static nl_args make_nl(etd_ctx *c) {
   a.bxo = a.bx * c->N;
   a.byo = a.by * c->N;
   a.bzo = a.bz * c->N;
+  a.ev = c->el_mix ? c->dconst->ev : nullptr;
   return a;
 }
 
@@ -1430,13 +1550,22 @@ void launch_nonlinear(etd_ctx *c, T *out, const T *sub, int ch_centre) {
     const int aniso = c->p.anisotropic;
     // with F2 the felas and ETD2 subtraction move to the divergence pass
     const T *sb = aniso ? nullptr : sub;
+    // (el_mix: every field's force needs the same six values, so it is taken
+    // here, once, also ahead of F2)
     const int fl = felas && !aniso;
     // FP32: all fields' loads at once; FP64 loads move twice the bytes, and
     // batches of 4 keep 8 waves per SIMD
     int fb = c->nl_batch;
     if (!fb) fb = sizeof(T) == 8 ? 4 : (c->nac <= 4 ? 4 : c->nac <= 8 ? 8 : c->nac <= 12 ? 12 : 16);
     const int mh = aniso ? 0 : 1;  // the grain mask goes with the last pass over the field
-    if (fb == 4)
+    if (felas && c->el_mix) {
+      if (c->nac <= 8)
+        k_nonlin_mix<T, 8><<<nb, 256, 0, c->stream>>>(F.u, out, sb, F.E, a, mh, a.ev);
+      else if (c->nac <= 12)
+        k_nonlin_mix<T, 12><<<nb, 256, 0, c->stream>>>(F.u, out, sb, F.E, a, mh, a.ev);
+      else
+        k_nonlin_mix<T, 16><<<nb, 256, 0, c->stream>>>(F.u, out, sb, F.E, a, mh, a.ev);
+    } else if (fb == 4)
       k_nonlin_ac<T, 4><<<nb, 256, 0, c->stream>>>(F.u, out, sb, F.E, a, fl, mh);
     else if (fb == 8)
       k_nonlin_ac<T, 8><<<nb, 256, 0, c->stream>>>(F.u, out, sb, F.E, a, fl, mh);
@@ -1444,16 +1573,17 @@ void launch_nonlinear(etd_ctx *c, T *out, const T *sub, int ch_centre) {
       k_nonlin_ac<T, 12><<<nb, 256, 0, c->stream>>>(F.u, out, sb, F.E, a, fl, mh);
     else
       k_nonlin_ac<T, 16><<<nb, 256, 0, c->stream>>>(F.u, out, sb, F.E, a, fl, mh);
+    const int felas2 = felas && !c->el_mix;
     if (aniso == 1)
       for (int p = 0; p < c->nac; p++) {
         k_f2_grad<T><<<round8(nb), 256, 0, c->stream>>>(F.u + n3 * p, F.gtmp, c->lam + 9 * p, a);
-        k_f2_div<T><<<round8(nb), 256, 0, c->stream>>>(F.gtmp, out + n3 * p, F.E, a, p, felas, F.u + n3 * p);
+        k_f2_div<T><<<round8(nb), 256, 0, c->stream>>>(F.gtmp, out + n3 * p, F.E, a, p, felas2, F.u + n3 * p);
         if (sub) launch_sub(c, out + n3 * p, sub + n3 * p, n3);  // after the F2 / felas terms
       }
     if (aniso == 2)
       for (int p = 0; p < c->nac; p++)
         k_f2_full<T><<<round8(nb), 256, 0, c->stream>>>(F.u + n3 * p, out + n3 * p, sub ? sub + n3 * p : nullptr,
-                                                        F.E, c->lam + 9 * p, a, p, felas);
+                                                        F.E, c->lam + 9 * p, a, p, felas2);
   }
   if (c->p.variable_mobility)
     launch_vm<T>(c, F.u, out, sub, F.gtmp, a);
@@ -1709,11 +1839,23 @@ struct fft16_cfg {
 // output goes to the felas ring, real and imaginary parts to the slots of
 // fields 2r and 2r+1, times 1/N^3 (the unpack); each value is rounded as the
 // separate pack / unpack kernels round it.
+// IO = 3, 4: the same with el_mix.  The pack forms the strain components
+// 2r, 2r + 1 from every field; the three pairs of a group of lines go to one
+// XCD one after another, so that the fields are read from HBM once (18 field
+// passes of bytes for 12 fields: 250 us FP64, 159 us FP32 at N = 192, 4.1
+// and 3.2 TB/s).  The unpack
+// keeps what it overwrites on the box edges (edge_cell) for the next
+// evaluation's lagged ghost cells.
 struct fft_io {
   const void *u;
   void *E;
   int n, g, nac, ring, slot0;
+  const double *ev;
 };
+// two or three coordinates of interior cell (x, y, z) lie within g of the box of edge N
+__device__ __forceinline__ bool edge_cell(int x, int y, int z, int N, int g) {
+  return (x < g || x >= N - g) + (y < g || y >= N - g) + (z < g || z >= N - g) >= 2;
+}
 
 template <int SGN, int R2, typename T2, int IO = 0>
 __global__ __launch_bounds__(256) void k_fft16(T2 *data, size_t fs, int axis, const double2 *__restrict__ tw,
@@ -1726,7 +1868,13 @@ __global__ __launch_bounds__(256) void k_fft16(T2 *data, size_t fs, int axis, co
   // the LDS, so twice the workgroups per CU) and FP64 pairs for FP64 data
   using LT = typename std::conditional<sizeof(T2) == 8, float2, double2>::type;
   __shared__ LT buf[16 * CF::LINE];
-  T2 *d = data + fs * blockIdx.y;
+  unsigned pr = blockIdx.y, bx = blockIdx.x;
+  if constexpr (IO == 3) {  // gridDim.x = 3 N^2 / 16
+    const unsigned t = blockIdx.x >> 3;
+    pr = t % 3;
+    bx = t / 3 * 8 + (blockIdx.x & 7);
+  }
+  T2 *d = data + fs * pr;
   const int tid = threadIdx.x;
   const int ll = axis == 0 ? tid >> 4 : tid & 15;  // line within the group
   const int j = axis == 0 ? tid & 15 : tid >> 4;   // thread within the line
@@ -1735,8 +1883,7 @@ __global__ __launch_bounds__(256) void k_fft16(T2 *data, size_t fs, int axis, co
   // Workgroups go to the 8 XCDs in turn and each XCD has its own L2, so there
   // each XCD takes a contiguous range of line groups (gridDim.x = N^2 / 16 is
   // a multiple of 8): both halves of a line meet in one L2.
-  unsigned bx = blockIdx.x;
-  if constexpr (IO == 2 && sizeof(T2) == 8) bx = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  if constexpr ((IO == 2 || IO == 4) && sizeof(T2) == 8) bx = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
   const unsigned L = bx * 16 + ll;                  // N^2 % 16 == 0: every line exists
   const unsigned x = L % N, o = L / N;
   const size_t base = axis == 0 ? (size_t)L * N : (axis == 1 ? x + (size_t)N * N * o : x + (size_t)N * o);
@@ -1745,7 +1892,7 @@ __global__ __launch_bounds__(256) void k_fft16(T2 *data, size_t fs, int axis, co
   {  // stage 1: thread n1 = j, DFT over n2 of x[n1 + 16 n2], twiddle, to LDS [k2][n1]
     const int n1 = j;
     double2 a[R2];
-    if constexpr (IO == 1) {
+    if constexpr (IO == 1 || IO == 3) {
       // axis 0, pack: the group's 16 x rows of fields 2r and 2r+1 go to LDS
       // with consecutive threads on consecutive x (coalesced; the rows of the
       // extended layout start two ghost cells in), padded so that the strided
@@ -1755,17 +1902,46 @@ __global__ __launch_bounds__(256) void k_fft16(T2 *data, size_t fs, int axis, co
       T2 *stg = reinterpret_cast<T2 *>(buf);
       const T *u = (const T *)io.u;
       const size_t n3 = (size_t)io.n * io.n * io.n;
-      const int pa = 2 * (int)blockIdx.y, pb = pa + 1;
+      const int pa = 2 * (int)pr, pb = pa + 1;
       // 16 N / 256 = R2 elements per thread, all loads issued before any
       // store (the loop is unrolled)
       T va[R2], vb[R2];
+      if constexpr (IO == 3) {
+        unsigned src[R2];
+        double sa[R2], sb[R2];
 #pragma unroll
-      for (int k = 0; k < R2; k++) {
-        const int e = tid + 256 * k, l2 = e / N, xx = e - l2 * N;
-        const unsigned Lg = bx * 16 + l2;
-        const size_t src = IDX(io.n, (int)(Lg / N) + io.g, (int)(Lg % N) + io.g, xx + io.g);
-        va[k] = u[n3 * pa + src];
-        vb[k] = pb < io.nac ? u[n3 * pb + src] : (T)0;
+        for (int k = 0; k < R2; k++) {
+          const int e = tid + 256 * k, l2 = e / N, xx = e - l2 * N;
+          const unsigned Lg = bx * 16 + l2;
+          src[k] = (unsigned)IDX(io.n, (int)(Lg / N) + io.g, (int)(Lg % N) + io.g, xx + io.g);
+          sa[k] = sb[k] = 0.0;
+        }
+        for (int q = 0; q < io.nac; q++) {
+          const T *uq = u + n3 * q;
+          const double ea = io.ev[6 * q + pa], eb = io.ev[6 * q + pb];
+          T v[R2];
+#pragma unroll
+          for (int k = 0; k < R2; k++) v[k] = uq[src[k]];
+#pragma unroll
+          for (int k = 0; k < R2; k++) {
+            sa[k] += ea * (double)v[k];
+            sb[k] += eb * (double)v[k];
+          }
+        }
+#pragma unroll
+        for (int k = 0; k < R2; k++) {
+          va[k] = (T)sa[k];
+          vb[k] = (T)sb[k];
+        }
+      } else {
+#pragma unroll
+        for (int k = 0; k < R2; k++) {
+          const int e = tid + 256 * k, l2 = e / N, xx = e - l2 * N;
+          const unsigned Lg = bx * 16 + l2;
+          const size_t src = IDX(io.n, (int)(Lg / N) + io.g, (int)(Lg % N) + io.g, xx + io.g);
+          va[k] = u[n3 * pa + src];
+          vb[k] = pb < io.nac ? u[n3 * pb + src] : (T)0;
+        }
       }
 #pragma unroll
       for (int k = 0; k < R2; k++) {
@@ -1817,11 +1993,21 @@ __global__ __launch_bounds__(256) void k_fft16(T2 *data, size_t fs, int axis, co
       v.x = b[k1].x;
       v.y = b[k1].y;
       const size_t m = base + (size_t)(k2 + R2 * k1) * stride;
-      if constexpr (IO == 2) {
+      if constexpr (IO == 4) {
+        const size_t N3 = (size_t)N * N * N;
+        const double inv = 1.0 / ((double)N * N * N);
+        T *E = (T *)io.E + (size_t)(2 * pr) * N3 + m;
+        if (edge_cell((int)x, (int)o, k2 + R2 * k1, N, io.g)) {
+          E[6 * N3] = E[0];
+          E[7 * N3] = E[N3];
+        }
+        E[0] = (T)((double)v.x * inv);
+        E[N3] = (T)((double)v.y * inv);
+      } else if constexpr (IO == 2) {
         T *E = (T *)io.E;
         const size_t N3 = (size_t)N * N * N;
         const double inv = 1.0 / ((double)N * N * N);
-        const int r = (int)blockIdx.y;
+        const int r = (int)pr;
         int sa = io.slot0 + 2 * r, sb = sa + 1;  // (slot0 + p) mod ring, p < nac < ring
         if (sa >= io.ring) sa -= io.ring;
         if (sb >= io.ring) sb -= io.ring;
@@ -1850,6 +2036,7 @@ static bool launch_fft16(etd_ctx *c, T2 *data, int npair, int axis, fft_io io = 
   const int N = c->Ne;
   if (!fft16_supported(N)) return false;
   dim3 grid((unsigned)((size_t)N * N / 16), npair);
+  if (IO == 3) grid = dim3(3 * (unsigned)((size_t)N * N / 16));  // npair is 3
   const double2 *tw = (const double2 *)c->tw;
   switch (N / 16) {
 #define F16(R)                                                                                   \
@@ -1924,6 +2111,37 @@ __global__ void k_el_pack_boxes(const T *__restrict__ u, typename cplx<T>::t *__
   zz.x = u[n3 * pa + src];
   zz.y = pb < nac ? u[n3 * pb + src] : (T)0;
   Z[N3 * r + m] = zz;
+}
+
+// el_mix: the six strain components of a point from every field, one box or
+// px per axis of edge N (the same addressing)
+template <typename T>
+__global__ __launch_bounds__(256) void k_el_pack_mix(const T *__restrict__ u, typename cplx<T>::t *__restrict__ Z,
+                                                     int n, int g, int N, int nac, int px, long long bs,
+                                                     const double *__restrict__ ev) {
+  const int Ng = px * N;
+  const size_t N3 = (size_t)Ng * Ng * Ng;
+  const size_t m = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (m >= N3) return;
+  int x, y, z;
+  idx3(m, Ng, x, y, z);
+  const size_t n3 = (size_t)n * n * n;
+  const int b = ((z / N) * px + y / N) * px + x / N;
+  const T *p = u + b * bs + (long long)IDX(n, z % N + g, y % N + g, x % N + g);
+  double s[6] = {0, 0, 0, 0, 0, 0};
+#pragma unroll 4
+  for (int q = 0; q < nac; q++) {
+    const double v = p[n3 * q];
+#pragma unroll
+    for (int a = 0; a < 6; a++) s[a] += ev[6 * q + a] * v;
+  }
+#pragma unroll
+  for (int r = 0; r < 3; r++) {
+    typename cplx<T>::t zz;
+    zz.x = (T)s[2 * r];
+    zz.y = (T)s[2 * r + 1];
+    Z[N3 * r + m] = zz;
+  }
 }
 
 // k-space contraction acc_p = sum_q B_pq(n) F_q with B computed on the fly
@@ -2162,6 +2380,37 @@ __global__ void k_el_unpack(const typename cplx<T>::t *__restrict__ Y, T *__rest
   if (2 * r + 1 < nac) E[(size_t)sb * N3 + m] = (T)((double)v.y * inv);
 }
 
+// el_mix: the stress components; what they overwrite stays on the edges of
+// the boxes of edge Nb
+template <typename T>
+__global__ void k_el_unpack_mix(const typename cplx<T>::t *__restrict__ Y, T *__restrict__ E, int N, int Nb, int g) {
+  const size_t N3 = (size_t)N * N * N;
+  const size_t m = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (m >= N3) return;
+  const int r = blockIdx.y;
+  int x, y, z;
+  idx3(m, N, x, y, z);
+  const double inv = 1.0 / ((double)N * N * N);
+  const typename cplx<T>::t v = Y[N3 * r + m];
+  T *e = E + (size_t)(2 * r) * N3 + m;
+  if (edge_cell(x % Nb, y % Nb, z % Nb, Nb, g)) {
+    e[6 * N3] = e[0];
+    e[7 * N3] = e[N3];
+  }
+  e[0] = (T)((double)v.x * inv);
+  e[N3] = (T)((double)v.y * inv);
+}
+
+// elastic_calculate (elastic.c:689-762): felas_p = IFFT(sum_q B_pq FFT(eta_q)).
+// B_pq is bilinear in the variants' eigenstrains, B_pq = sum_ab ev_pa B_ab
+// ev_qb over the six components of a symmetric strain, so with more than six
+// variants (el_mix) the six fields g_a = sum_q ev_qa eta_q are transformed,
+// contracted with the B of the six unit strains and transformed back, and
+// felas_p = sum_a ev_pa G_a is formed where it is used: 3 packed transforms
+// each way instead of 6 for 12 variants, and 6 fields to read in the
+// nonlinear term instead of 12.  Up to six variants it saves nothing.
+// 192^3 x 12, a step's elasticity: 2.08 -> 1.17 ms FP64, 1.13 -> 0.64 ms
+// FP32, and its nonlinear terms 0.48 -> 0.37 and 0.29 -> 0.24 ms.
 template <typename T>
 void launch_elastic(etd_ctx *c) {
   using T2 = typename cplx<T>::t;
@@ -2178,15 +2427,22 @@ void launch_elastic(etd_ctx *c) {
   // (the fused passes exist only where the two-stage kernel does: N = 16 R2
   // with an instantiated R2; elsewhere pack, radix passes and unpack)
   const bool fused = c->fft_variant == 1 && fft16_supported(N) && c->P == 1;
-  fft_io io{uel, F.E, c->n, c->g, c->nel, c->ring, slot0};
+  const double *ev = c->el_mix ? c->dconst->ev : nullptr;
+  fft_io io{uel, F.E, c->n, c->g, c->nel, c->ring, slot0, ev};
   if (fused) {
     etd_prof_begin(c, PC_FFT);
-    launch_fft16<1, T2, 1>(c, (T2 *)F.Z, c->npair, 0, io);
+    if (c->el_mix)
+      launch_fft16<1, T2, 3>(c, (T2 *)F.Z, c->npair, 0, io);
+    else
+      launch_fft16<1, T2, 1>(c, (T2 *)F.Z, c->npair, 0, io);
     launch_fft16<1, T2>(c, (T2 *)F.Z, c->npair, 1);
     launch_fft16<1, T2>(c, (T2 *)F.Z, c->npair, 2);
     etd_prof_end(c, PC_FFT);
   } else {
-    if (c->P == 1)
+    if (c->el_mix)
+      k_el_pack_mix<T><<<nb, 256, 0, c->stream>>>(uel, (T2 *)F.Z, c->n, c->g, c->N, c->nel, c->P == 1 ? 1 : c->px,
+                                                  (long long)c->bs, ev);
+    else if (c->P == 1)
       k_el_pack<T><<<dim3(nb, c->npair), 256, 0, c->stream>>>(uel, (T2 *)F.Z, c->n, c->g, N, c->nel);
     else
       k_el_pack_boxes<T><<<dim3(nb, c->npair), 256, 0, c->stream>>>(uel, (T2 *)F.Z, c->n, c->g, c->N, c->nel, c->px,
@@ -2199,7 +2455,7 @@ void launch_elastic(etd_ctx *c) {
     const unsigned nbh = (unsigned)(((size_t)N * N * (N / 2 + 1) + 255) / 256);
     const T2 *Zc = (const T2 *)F.Z;
     T2 *Yc = (T2 *)F.Y;
-    switch (c->nel) {
+    switch (c->nft) {
 #define NACC(X)                                                                                    case X:                                                                                            k_el_contract_t<X, T2><<<nbh, 256, 0, c->stream>>>(Zc, Yc, N, c->npair, c->dconst);                  k_el_contract_mirror<X, T2><<<nbm, 256, 0, c->stream>>>(Zc, Yc, N, c->npair, c->dconst);            break;
       NACC(1) NACC(2) NACC(3) NACC(4) NACC(5) NACC(6) NACC(7) NACC(8) NACC(9) NACC(10) NACC(11) NACC(12) NACC(13)
       NACC(14) NACC(15) NACC(16)
@@ -2211,8 +2467,14 @@ void launch_elastic(etd_ctx *c) {
     etd_prof_begin(c, PC_FFT);
     launch_fft16<-1, T2>(c, (T2 *)F.Y, c->npair, 0);
     launch_fft16<-1, T2>(c, (T2 *)F.Y, c->npair, 1);
-    launch_fft16<-1, T2, 2>(c, (T2 *)F.Y, c->npair, 2, io);
+    if (c->el_mix)
+      launch_fft16<-1, T2, 4>(c, (T2 *)F.Y, c->npair, 2, io);
+    else
+      launch_fft16<-1, T2, 2>(c, (T2 *)F.Y, c->npair, 2, io);
     etd_prof_end(c, PC_FFT);
+  } else if (c->el_mix) {
+    fft3d<T>(c, F.Y, c->npair, -1);
+    k_el_unpack_mix<T><<<dim3(nb, c->npair), 256, 0, c->stream>>>((const T2 *)F.Y, F.E, N, c->N, c->g);
   } else {
     fft3d<T>(c, F.Y, c->npair, -1);
     k_el_unpack<T><<<dim3(nb, c->npair), 256, 0, c->stream>>>((const T2 *)F.Y, F.E, N, c->nel, c->ring, slot0);
