@@ -199,6 +199,7 @@ extern "C" int etd_create(const etd_params *p, const double *Vh, const double *V
   c->mp_nb = 8;
   const char *cv = getenv("ETD_CARRY");
   c->no_carry = cv && atoi(cv) == 0;  // every step transforms u itself
+  c->carry_always = cv && atoi(cv) == 1;
   carry_base(c, nullptr, 1.0, nullptr, 0.0);
   c->fft_variant = 1;
   const char *fv = getenv("ETD_FFT");

@@ -197,11 +197,30 @@ static size_t carry_elems(const etd_ctx *c, size_t *off) {
   return o;
 }
 
-// one box, two ghost layers, and coefficients whose exp(-dt H) factors stay
+// Whether carrying pays.  It saves three field passes of the mode products
+// per AC field and costs the correction: two batched GEMMs, the axis factors
+// and a pass whose blocks are few and long on small boxes (19 us at n = 36).
+// FP64, fixed ETD1 steps without elasticity, carried against transforming u:
+// n = 36 x 4 fields 70 / 47 us, 68 x 4 112 / 89, 100 x 4 198 / 194, 116 x 4
+// 282 / 289, 84 x 12 367 / 358, 100 x 12 561 / 572, 132 x 1 178 / 171,
+// 164 x 1 249 / 283, 196 x 12 4152 / 5032: the line lies near n^3 sqrt(nac) =
+// 2.7e6.  ETD2 corrects twice a step: 132 x 12 2520 / 2365, 164 x 12 4854 /
+// 4881, 196 x 4 2764 / 2767, 260 x 4 6792 / 7178.  With physical sides there
+// are no GEMMs: 68 x 4 81 / 82, ETD2 68 x 4 164 / 155, 100 x 4 317 / 341.
+// The mixed path carries at any size: it is the more accurate of the two
+// there (u is not rounded by a transform of its own every step).
+static bool carry_pays(const etd_ctx *c) {
+  if (c->mixed || c->carry_always) return true;
+  const double m = (double)c->n3 * sqrt((double)c->nac);
+  if (!c->p.periodic) return m >= (c->p.etd2 ? 1.5e6 : 0.6e6);
+  return m >= (c->p.etd2 ? 15e6 : 2.7e6);
+}
+
+// one box, two ghost layers, a size at which it pays, and coefficients whose exp(-dt H) factors stay
 // at most 1 (k_phi_axes)
 bool carry_possible(const etd_ctx *c) {
   const etd_params &p = c->p;
-  return c->P == 1 && c->nac > 0 && c->g == 2 && !c->no_carry && p.LE >= 0 && p.epn2 >= 0 && p.kkx >= 0 &&
+  return c->P == 1 && c->nac > 0 && c->g == 2 && !c->no_carry && carry_pays(c) && p.LE >= 0 && p.epn2 >= 0 && p.kkx >= 0 &&
          p.kky >= 0 && p.kkz >= 0;
 }
 

@@ -146,6 +146,7 @@ struct etd_ctx {
    * and nothing has changed u since; no_carry turns it off (ETD_CARRY=0,
    * ensemble members); cr_buf the correction's buffers */
   int carry_ok, no_carry;
+  int carry_always;        /* ETD_CARRY=1: carry also where it does not pay (carry_pays) */
   const void *carry_s1, *carry_s2;
   double carry_alpha, carry_beta;
   /* set by stage_forward: the AC spectrum still lacks the fill's changes,
