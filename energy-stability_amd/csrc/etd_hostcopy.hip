@@ -28,7 +28,11 @@
 #define HC_SHARE ((size_t)8 << 20)   // host bytes that pay for one more thread (from two on)
 #define HC_SLOTS 3
 #define HC_MIN ((size_t)64 << 10)    // least device bytes per slot
-#define HC_DIRECT ((size_t)1 << 20)  // FP64 up to this: the runtime's own path
+// FP64 fields up to this: the runtime's own path (n = 68, read 147 us there,
+// 142 here, set 100 and 128; n = 84 read 273 and 222, set 148 and 190; n = 100
+// set 236 and 258, n = 132 set 506 and 490)
+#define HC_DIRECT_GET ((size_t)3 << 20)
+#define HC_DIRECT_PUT ((size_t)8 << 20)
 
 // host FP64 values from device ones, past the cache for long runs
 static void widen(double *dst, const double *src, size_t cnt) { memcpy(dst, src, sizeof(double) * cnt); }
@@ -245,7 +249,7 @@ static hipError_t hc_plain(etd_ctx *c, float *dev, double *host, size_t cnt, int
 template <typename T>
 hipError_t host_copy(etd_ctx *c, T *dev, double *host, size_t cnt, int put) {
   const size_t bytes = sizeof(T) * cnt;
-  if (sizeof(T) == 8 && bytes <= HC_DIRECT) return hc_plain(c, dev, host, cnt, put);
+  if (sizeof(T) == 8 && bytes <= (put ? HC_DIRECT_PUT : HC_DIRECT_GET)) return hc_plain(c, dev, host, cnt, put);
   // a quarter of the field per chunk, at most HC_CHUNK, in whole 4 KiB; half
   // of it up to 4 MiB (quarters that short took 430 us from the device at
   // 1 MiB, halves 70 us)

@@ -137,6 +137,98 @@ __global__ void k_ghost_x(T *base, size_t fs, int n, int g, long long lo, long l
   u[IDX(n, k, j, i)] = v;
 }
 
+// The three sweeps of one box in one launch.  A cell's value depends on the
+// pre-transfer state only, so the work is cut such that whoever reads a cell
+// that changes also writes it: the row (k, j) of an interior plane and, where
+// k or j is the source of ghost planes or rows, its copies
+//   (kg, j), (k, jg), (kg, jg)    kg, jg the ghosts of k, j
+// belong to one wave, which reads both rows it needs (k, j) and (k, jg) before
+// it writes any: z takes the whole row, y the row of an interior plane, x what
+// is left.  Rows that are no source have only their 2g x ghosts to fill: a
+// thread each.  Blocks [0, nrow) take the former, four rows each, the rest
+// the latter.  A step's fills, three launches against one: FP64 x 4, n = 36
+// 11.2 / 6.5 us, n = 196 26.6 / 23.9; FP64 x 13, n = 100 31.9 / 22.8, n = 196
+// 72.5 / 61.2 (the AC fields' and the CH field's fill).
+template <typename T>
+__global__ __launch_bounds__(256) void k_ghost_fill(T *base, size_t fs, int n, int g, unsigned nrow, T *dz, T *dy,
+                                                    T *dx) {
+  T *u = base + fs * blockIdx.y;
+  const int m = n - 2 * g, G = 2 * g;
+  const size_t n2 = (size_t)n * n, fd = (size_t)G * n2 * blockIdx.y;
+  // interior coordinate e is the source of a ghost when it lies within g of
+  // an end: ghost e + m from the low end, e - m from the high end (m >= 2g:
+  // not both); its index among the 2g ghost layers
+  auto ghost_of = [&](int e) { return e < G ? e + m : e >= m ? e - m : -1; };
+  auto layer_of = [&](int e) { return e < g ? e : e - n + G; };
+  if (blockIdx.x < nrow) {
+    // source rows: planes k that are sources (2g of them) x all m rows, then
+    // the other planes x their 2g source rows
+    const int r = (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    int k, j;
+    if (r < G * m) {
+      const int q = r / m;
+      k = q < g ? g + q : m + q - g;  // g .. 2g-1, m .. m+g-1
+      j = g + r - q * m;
+    } else {
+      const int r2 = r - G * m, q = r2 / G, s = r2 - q * G;
+      if (q >= m - G) return;
+      k = G + q;
+      j = s < g ? g + s : m + s - g;
+    }
+    const int kg = ghost_of(k), jg = ghost_of(j);
+    // n <= 272: five cells of each row per lane
+    T a[5], b[5];
+#pragma unroll
+    for (int c = 0; c < 5; c++) {
+      const int i = lane + 64 * c;
+      if (i < n) {
+        a[c] = u[IDX(n, k, j, i)];
+        if (jg >= 0) b[c] = u[IDX(n, k, jg, i)];
+      }
+    }
+    // the x ghosts of row (k, j): its interior cells one period away
+    T xv = 0, xo = 0;
+    int xi = 0;
+    if (lane < G) {
+      xi = lane < g ? lane : n - G + lane;
+      xv = u[IDX(n, k, j, wrap_e(xi, n, g))];
+      xo = u[IDX(n, k, j, xi)];
+    }
+    auto put = [&](size_t to, size_t rec, T *dlt, T v) {
+      if (dlt) dlt[fd + rec] = (T)((double)v - (double)u[to]);
+      u[to] = v;
+    };
+    // every lane's reads of the two rows come before any lane's writes: one wave runs in step
+#pragma unroll
+    for (int c = 0; c < 5; c++) {
+      const int i = lane + 64 * c;
+      if (i < n) {
+        if (kg >= 0) put(IDX(n, kg, j, i), (size_t)layer_of(kg) * n2 + (size_t)j * n + i, dz, a[c]);
+        if (kg >= 0 && jg >= 0) put(IDX(n, kg, jg, i), (size_t)layer_of(kg) * n2 + (size_t)jg * n + i, dz, b[c]);
+        if (jg >= 0) {
+          if (dy) dy[fd + ((size_t)layer_of(jg) * n + k) * n + i] = (T)((double)a[c] - (double)b[c]);
+          u[IDX(n, k, jg, i)] = a[c];
+        }
+      }
+    }
+    if (lane < G) {
+      if (dx) dx[fd + ((size_t)lane * n + k) * n + j] = (T)((double)xv - (double)xo);
+      u[IDX(n, k, j, xi)] = xv;
+    }
+    return;
+  }
+  const int w = m - G;  // planes, and rows of a plane, that are no source
+  const unsigned t = (blockIdx.x - nrow) * 256u + threadIdx.x;
+  if (t >= (unsigned)(w * w * G)) return;
+  const unsigned row = t / (unsigned)G;
+  const int cc = (int)(t - row * (unsigned)G);
+  const int k = G + (int)(row / (unsigned)w), j = G + (int)(row % (unsigned)w);
+  const int i = cc < g ? cc : n - G + cc;
+  const T v = u[IDX(n, k, j, wrap_e(i, n, g))];
+  if (dx) dx[fd + ((size_t)cc * n + k) * n + j] = (T)((double)v - (double)u[IDX(n, k, j, i)]);
+  u[IDX(n, k, j, i)] = v;
+}
+
 // element offset from box b's fields to those of the box (sx, sy, sz) away
 static long long host_box_off(const etd_ctx *c, int b, int sx, int sy, int sz) {
   const int bx = b % c->px, by = (b / c->px) % c->py, bz = b / (c->px * c->py);
@@ -153,6 +245,18 @@ void launch_ghost_fill(etd_ctx *c, T *base, int nfields, size_t fstride, T *dz, 
   const size_t n2 = (size_t)n * n;
   size_t tz = 2 * g * n2, ty = (size_t)(n - 2 * g) * 2 * g * n, tx = (size_t)(n - 2 * g) * (n - 2 * g) * 2 * g;
   etd_prof_begin(c, PC_HALO);
+  const int m = n - 2 * g, w = m - 2 * g;
+  // one launch for one box whose interior holds both ends' source layers
+  // apart, rows of at most 5 x 64 cells, 2g <= 64 x ghosts; the sweeps
+  // otherwise (a decomposed run's boxes read each other's ghost cells)
+  if (c->P == 1 && w >= 0 && n <= 320 && 2 * g <= 64) {
+    const size_t rows = (size_t)2 * g * m + (size_t)w * 2 * g, xs = (size_t)w * w * 2 * g;
+    const unsigned nrow = (unsigned)((rows + 3) / 4);
+    k_ghost_fill<T><<<dim3(nrow + (unsigned)((xs + 255) / 256), nfields), 256, 0, c->stream>>>(base, fstride, n, g,
+                                                                                             nrow, dz, dy, dx);
+    etd_prof_end(c, PC_HALO);
+    return;
+  }
   for (int b = 0; b < c->P; b++)
     k_ghost_z<T><<<dim3((unsigned)((tz + 255) / 256), nfields), 256, 0, c->stream>>>(
         base + b * c->bs, fstride, n, g, host_box_off(c, b, 0, 0, -1), host_box_off(c, b, 0, 0, 1), dz);
@@ -2329,27 +2433,35 @@ __device__ __forceinline__ void contract_point(const T2 *__restrict__ Z, T2 *__r
 // One thread per pair {k, -k}: planes z = 0 .. N/2 hold a member of every
 // pair; the point with the smaller index computes both (within the planes
 // z = 0 and z = N/2, which map to themselves, half the threads return).
-template <int NAC, typename T2>
-__global__ __launch_bounds__(256) void k_el_contract_t(const T2 *__restrict__ Z, T2 *__restrict__ Y, int N,
-                                                       int npair, const etd_dev_consts *__restrict__ K) {
-  const size_t m = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+// SKIP: leave the mirror points out.
+template <int NAC, bool SKIP, typename T2>
+__device__ __forceinline__ void contract_pair(const T2 *__restrict__ Z, T2 *__restrict__ Y, int N, int npair, size_t m,
+                                              const etd_dev_consts *__restrict__ K) {
   if (m >= (size_t)N * N * (N / 2 + 1)) return;
   int x, y, z;
   idx3(m, N, x, y, z);
   const int xm = (N - x) % N, ym = (N - y) % N, zm = (N - z) % N;
   if (((size_t)zm * N + ym) * N + xm < m) return;
+  if constexpr (SKIP) {
+    const int c = N / 2, d = c + (N & 1);
+    if (x == c || x == d || y == c || y == d || z == c || z == d) return;
+  }
   contract_point<NAC, false, T2, true>(Z, Y, N, npair, m, K);
+}
+template <int NAC, typename T2>
+__global__ __launch_bounds__(256) void k_el_contract_t(const T2 *__restrict__ Z, T2 *__restrict__ Y, int N,
+                                                       int npair, const etd_dev_consts *__restrict__ K) {
+  contract_pair<NAC, false, T2>(Z, Y, N, npair, (size_t)blockIdx.x * blockDim.x + threadIdx.x, K);
 }
 
 // points whose mirror's signed wavenumber is not the negative: the index
 // planes c = N/2 (and c = N/2 + 1 for odd N) in each direction; one thread
 // per (plane, position), duplicates across the planes write equal values
 template <int NAC, typename T2>
-__global__ __launch_bounds__(256) void k_el_contract_mirror(const T2 *__restrict__ Z, T2 *__restrict__ Y,
-                                                            int N, int npair, const etd_dev_consts *__restrict__ K) {
+__device__ __forceinline__ void contract_mirror(const T2 *__restrict__ Z, T2 *__restrict__ Y, int N, int npair,
+                                                size_t t, const etd_dev_consts *__restrict__ K) {
   const int nplane = (N & 1) ? 2 : 1;
   const size_t N2 = (size_t)N * N;
-  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= 3 * nplane * N2) return;
   const int axis = (int)(t / (nplane * N2));
   const int which = (int)((t / N2) % nplane);
@@ -2361,6 +2473,29 @@ __global__ __launch_bounds__(256) void k_el_contract_mirror(const T2 *__restrict
   else if (axis == 1) { x = a; y = c; z = b; }
   else { x = a; y = b; z = c; }
   contract_point<NAC, true, T2>(Z, Y, N, npair, ((size_t)z * N + y) * N + x, K);
+}
+template <int NAC, typename T2>
+__global__ __launch_bounds__(256) void k_el_contract_mirror(const T2 *__restrict__ Z, T2 *__restrict__ Y,
+                                                            int N, int npair, const etd_dev_consts *__restrict__ K) {
+  contract_mirror<NAC, T2>(Z, Y, N, npair, (size_t)blockIdx.x * blockDim.x + threadIdx.x, K);
+}
+
+// Both in one launch, the mirror points first (blocks [0, nbm), the longer
+// ones): each kernel by itself is one long chain on a small grid (8 us each at
+// N = 64, four FP64 variants), and on large ones the mirror points (38 us at
+// N = 192) run beside the others.  A step's elasticity, two launches against
+// one: FP64 x 4, N = 64 67.4 / 61.7 us, 96 113.5 / 106.6, 160 388 / 386, 192
+// 634.5 / 639; FP32 x 4, N = 64 59.3 / 53.8, 192 377.4 / 374.2; FP32 x 12 (six
+// transformed) N = 80 102.6 / 96.9, 192 634 / 628.  More variants (FP64 six,
+// FP32 seven) leave the joint kernel one wave per SIMD; they keep two.
+template <int NAC, typename T2>
+__global__ __launch_bounds__(256) void k_el_contract_one(const T2 *__restrict__ Z, T2 *__restrict__ Y, int N,
+                                                         int npair, const etd_dev_consts *__restrict__ K,
+                                                         unsigned nbm) {
+  if (blockIdx.x < nbm)
+    contract_mirror<NAC, T2>(Z, Y, N, npair, (size_t)blockIdx.x * 256 + threadIdx.x, K);
+  else
+    contract_pair<NAC, true, T2>(Z, Y, N, npair, (size_t)(blockIdx.x - nbm) * 256 + threadIdx.x, K);
 }
 
 template <typename T>
@@ -2455,8 +2590,19 @@ void launch_elastic(etd_ctx *c) {
     const unsigned nbh = (unsigned)(((size_t)N * N * (N / 2 + 1) + 255) / 256);
     const T2 *Zc = (const T2 *)F.Z;
     T2 *Yc = (T2 *)F.Y;
+    bool one = false;
     switch (c->nft) {
-#define NACC(X)                                                                                    case X:                                                                                            k_el_contract_t<X, T2><<<nbh, 256, 0, c->stream>>>(Zc, Yc, N, c->npair, c->dconst);                  k_el_contract_mirror<X, T2><<<nbm, 256, 0, c->stream>>>(Zc, Yc, N, c->npair, c->dconst);            break;
+#define NACC(X)                                                                                       \
+  case X:                                                                                             \
+    if constexpr (X <= (sizeof(T) == 4 ? 6 : 5)) one = sizeof(T) == 4 || N <= 168;                    \
+    if (one) {                                                                                        \
+      if constexpr (X <= 6)                                                                           \
+      k_el_contract_one<X, T2><<<nbm + nbh, 256, 0, c->stream>>>(Zc, Yc, N, c->npair, c->dconst, nbm); \
+    } else {                                                                                          \
+      k_el_contract_t<X, T2><<<nbh, 256, 0, c->stream>>>(Zc, Yc, N, c->npair, c->dconst);             \
+      k_el_contract_mirror<X, T2><<<nbm, 256, 0, c->stream>>>(Zc, Yc, N, c->npair, c->dconst);        \
+    }                                                                                                 \
+    break;
       NACC(1) NACC(2) NACC(3) NACC(4) NACC(5) NACC(6) NACC(7) NACC(8) NACC(9) NACC(10) NACC(11) NACC(12) NACC(13)
       NACC(14) NACC(15) NACC(16)
 #undef NACC
