@@ -98,7 +98,7 @@ struct etd_ctx {
   long long elastic_evals; /* completed elastic evaluations */
   int elastic_fresh;       /* the latest evaluation is of the current fields (adaptive energy test) */
   int fft_radix[16], fft_npass;
-  int fft_variant;         /* 1: two-stage register FFT for N % 16 == 0 (default), 0: radix passes in LDS */
+  int fft_variant;         /* 1: two-stage register FFT where N has one (default), 0: radix passes in LDS */
   int split_waves;         /* mixed mode products: 8 or 4 waves per workgroup, 0 by size */
   int split_persistent;    /* 1: persistent workgroups looping over tiles (default) */
   int split_kernel;        /* BF16 split-3: 0: field chunks staged through LDS, 8 waves x 32 columns;
@@ -291,7 +291,8 @@ int launch_diag(etd_ctx *c, double *stats);
 /* doubles of partial sums one check_soln_new evaluation writes (the size of c->part) */
 size_t etd_diag_partials(const etd_ctx *c);
 /* the two-stage register FFT (k_fft16) handles this N */
-bool fft16_supported(int N);
+bool fft16_supported(int N);  /* N = 16 R2 */
+bool fft2_supported(int N);   /* any two-stage transform (etd_fft2.hip) */
 /* CH mean conservation of the mixed path: ch_mean_mark takes the interior
  * sums of the CH fields of the state u (V fields, stride n3) as the targets
  * if the fields were set since the last mark; ch_mean_restore shifts the CH
