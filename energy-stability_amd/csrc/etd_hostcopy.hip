@@ -8,7 +8,7 @@
 // others convert (or copy) their share of each chunk that has arrived.
 // Measured, one field read (set), before against now: n = 196 FP64 3.4 (2.0)
 // -> 1.4 (1.4) ms, FP32 3.5 (2.7) -> 0.8 (0.8) ms; n = 260 FP32 21.8 (16.3)
-// -> 1.6 (1.7) ms; n = 36 FP32 88 -> 41 us.  Chunks: a copy costs about 13 us
+// -> 1.6 (1.7) ms; n = 36 FP32 21 to 90 -> 20 us.  Chunks: a copy costs about 13 us
 // besides its bytes, so 512 KiB pieces reach 21 GB/s, 4 MiB 43 GB/s; more
 // than 4 threads add nothing.
 #include <hip/hip_runtime.h>
@@ -33,6 +33,11 @@
 // set 236 and 258, n = 132 set 506 and 490)
 #define HC_DIRECT_GET ((size_t)3 << 20)
 #define HC_DIRECT_PUT ((size_t)8 << 20)
+// FP32 fields up to this: one copy through one slot, no events (read, two
+// chunks against one slot: n = 36 39 and 20 us, n = 52 49 and 35, n = 68 71 and
+// 66, n = 84 108 and 125; a temporary on the heap, as before the slots, 21 to
+// 90, 43, 104, 195)
+#define HC_ONE ((size_t)2 << 20)
 
 // host FP64 values from device ones, past the cache for long runs
 static void widen(double *dst, const double *src, size_t cnt) { memcpy(dst, src, sizeof(double) * cnt); }
@@ -223,16 +228,18 @@ static int hc_events(etd_ctx *c) {
   return 1;
 }
 
-// the copy without slots of its own: FP64 directly, FP32 through a temporary
-static hipError_t hc_plain(etd_ctx *c, double *dev, double *host, size_t cnt, int put) {
+// one copy: FP64 directly, FP32 through one slot, or the heap where pinned
+// memory cannot be had
+static hipError_t hc_one(etd_ctx *c, double *dev, double *host, size_t cnt, int put) {
   hipError_t e = put ? hipMemcpyAsync(dev, host, sizeof(double) * cnt, hipMemcpyHostToDevice, c->stream)
                      : hipMemcpyAsync(host, dev, sizeof(double) * cnt, hipMemcpyDeviceToHost, c->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
   return e;
 }
-static hipError_t hc_plain(etd_ctx *c, float *dev, double *host, size_t cnt, int put) {
-  float *t = (float *)malloc(sizeof(float) * cnt);
-  if (!t) return hipErrorOutOfMemory;
+static hipError_t hc_one(etd_ctx *c, float *dev, double *host, size_t cnt, int put) {
+  size_t pinned = 0;
+  float *pin = (float *)pool_take(sizeof(float) * cnt, &pinned), *t = pin;
+  if (!t && !(t = (float *)malloc(sizeof(float) * cnt))) return hipErrorOutOfMemory;
   hipError_t e = hipSuccess;
   if (put) {
     narrow(t, host, cnt);
@@ -242,14 +249,15 @@ static hipError_t hc_plain(etd_ctx *c, float *dev, double *host, size_t cnt, int
   }
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
   if (e == hipSuccess && !put) widen(host, t, cnt);
-  free(t);
+  if (pin) pool_give(pin, pinned);
+  else free(t);
   return e;
 }
 
 template <typename T>
 hipError_t host_copy(etd_ctx *c, T *dev, double *host, size_t cnt, int put) {
   const size_t bytes = sizeof(T) * cnt;
-  if (sizeof(T) == 8 && bytes <= (put ? HC_DIRECT_PUT : HC_DIRECT_GET)) return hc_plain(c, dev, host, cnt, put);
+  if (bytes <= (sizeof(T) == 4 ? HC_ONE : put ? HC_DIRECT_PUT : HC_DIRECT_GET)) return hc_one(c, dev, host, cnt, put);
   // a quarter of the field per chunk, at most HC_CHUNK, in whole 4 KiB; half
   // of it up to 4 MiB (quarters that short took 430 us from the device at
   // 1 MiB, halves 70 us)
@@ -258,7 +266,7 @@ hipError_t host_copy(etd_ctx *c, T *dev, double *host, size_t cnt, int put) {
   const size_t nch = (bytes + per - 1) / per;
   size_t pinned = 0;
   void *pin = hc_events(c) ? pool_take((nch < HC_SLOTS ? nch : HC_SLOTS) * per, &pinned) : nullptr;
-  if (!pin) return hc_plain(c, dev, host, cnt, put);
+  if (!pin) return hc_one(c, dev, host, cnt, put);
   hc_job<T> job;
   job.pin = pin;
   job.c = c;
