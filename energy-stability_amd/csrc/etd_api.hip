@@ -584,33 +584,6 @@ static void box_view(etd_ctx *c, int b) {
   c->box = b;
 }
 
-// the nonlinear terms of every box (out, sub: box 0's first field, the
-// others at stride bs); each box reads its neighbours' fields for the
-// outside values, so all boxes are evaluated before any is advanced
-template <typename T>
-static void nonlinear_boxes(etd_ctx *c, T *out, const T *sub, int ch_centre) {
-  if (c->P == 1) {
-    launch_nonlinear<T>(c, out, sub, ch_centre);
-    return;
-  }
-  if constexpr (sizeof(T) == 8) {
-    for (int b = 0; b < c->P; b++) {
-      box_view(c, b);
-      launch_nonlinear<T>(c, out + b * c->bs, sub ? sub + b * c->bs : nullptr, ch_centre);
-    }
-    box_view(c, 0);
-  }
-}
-
-// phi scaling of every box: u-hat of box b at spec + b bs, N-hat after all
-// boxes' u-hat (the forward transform's input was [u of all boxes | N1 of all])
-template <typename T>
-static void phiscale_boxes(etd_ctx *c, T *spec, const T *nhat0, int order2) {
-  const size_t bs = c->bs;
-  for (int b = 0; b < c->P; b++)
-    launch_phiscale<T>(c, spec + b * bs, nhat0 ? nhat0 + b * bs : nullptr, spec + b * bs, 0, c->V, order2);
-}
-
 // ------------------------------------------------------------------ step
 // Three rotating mode products by V^-1 (forward) or V (backward) over nf
 // fields; FP64 MFMA on the plain path, split-BF16 MFMA on the mixed path.
@@ -678,7 +651,7 @@ void stage_forward(etd_ctx *c) {
   // these fields (same ghost fill, same kernels): reuse it
   if (c->nel > 0 && !c->elastic_fresh) launch_elastic<T>(c);
   c->elastic_fresh = 0;
-  nonlinear_boxes<T>(c, F.N1, (const T *)nullptr, 1);  // mixed: CH terms centred, N1 - N(c_mean)
+  launch_nonlinear<T>(c, F.N1, (const T *)nullptr, 1);  // mixed: CH terms centred, N1 - N(c_mean)
   if constexpr (sizeof(T) == 4) ch_center(c, F.u, nullptr, -1);
   if (carry) {
     modeprod3<T>(c, 1, F.u + c->n3 * c->nac, F.spec + c->n3 * c->nac, c->nch + V, 0);
@@ -707,7 +680,8 @@ void phi_stage(etd_ctx *c, T *out, double dt, T *out2, double dt2) {
     if (out2)
       launch_phiscale_pair<T>(c, F.spec, nhat, out, dt, out2, dt2, 0, V);
     else
-      phiscale_boxes<T>(c, F.spec, nhat, 0);
+      // the forward transform's input was [u of all boxes | N1 of all]
+      launch_phiscale<T>(c, F.spec, nhat, F.spec, 0, V, 0, c->P);
     return;
   }
   c->carry_pend = 0;  // only single-box contexts carry: N-hat is at spec + n3 V
@@ -744,12 +718,12 @@ void etd2_stage(etd_ctx *c, const T *ahat, T *spec_out) {
     launch_ghost_fill<T>(c, F.u, V, n3);
   }
   if (c->nel > 0) launch_elastic<T>(c);
-  nonlinear_boxes<T>(c, F.N2, (const T *)F.N1, 0);  // N(a) - N(u_n)
+  launch_nonlinear<T>(c, F.N2, (const T *)F.N1, 0);  // N(a) - N(u_n)
   // the corrector's spectra in the N-hat half (free after the phi update),
   // so that a-hat stays where it is
   T *dsp = F.spec + n3 * PV;
   modeprod3<T>(c, 1, F.N2, dsp, PV, 0);
-  phiscale_boxes<T>(c, dsp, (const T *)nullptr, 1);
+  launch_phiscale<T>(c, dsp, (const T *)nullptr, dsp, 0, V, 1, c->P);
   modeprod3<T>(c, 0, dsp, F.u, PV, 1);  // u = a + S phi2 S^-1 dN
   if (spec_out) carry_correct<T>(c, ahat, 1.0, dsp, 1.0, spec_out);
   if constexpr (sizeof(T) == 4) ch_mean_restore(c, F.u);
@@ -952,7 +926,7 @@ extern "C" int etd_k_nonlinear(etd_ctx *c, int var, double *host_out) {
     HCHK(c, hipGetLastError());
     return get_f32(c, host_out, c->f32.N1 + c->n3 * var, c->n3);
   }
-  nonlinear_boxes<double>(c, c->N1, (const double *)nullptr, 0);
+  launch_nonlinear<double>(c, c->N1, (const double *)nullptr, 0);
   HCHK(c, hipGetLastError());
   for (int b = 0; b < c->P; b++)  // a decomposed run: the boxes one after another
     HCHK(c, hipMemcpyAsync(host_out + b * c->n3, c->N1 + b * c->bs + c->n3 * var, sizeof(double) * c->n3,

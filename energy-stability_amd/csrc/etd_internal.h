@@ -262,7 +262,8 @@ static inline phi_args phi_args_of(const etd_ctx *c, double dt, double dt2) {
   return a;
 }
 template <typename T>
-void launch_phiscale(etd_ctx *c, const T *uhat, const T *nhat, T *out, int first_var, int nvars, int order2);
+void launch_phiscale(etd_ctx *c, const T *uhat, const T *nhat, T *out, int first_var, int nvars, int order2,
+                     int boxes = 1);
 /* first order over fields first_var .. first_var + nvars (pointers at
  * field first_var): out at step dt, out2 at step dt2 */
 template <typename T>

@@ -93,9 +93,25 @@ __device__ __forceinline__ void idx3(size_t l, int n, int &i, int &j, int &k) {
 // field as 2g contiguous n x n matrices: z [plane][j][i], y [row][k][i], x
 // [column][k][j] (y and x write their interior rows / columns only; the
 // rest of their matrices stays zero).
+struct ghost_boxes {  // px x py x pz boxes, bs elements apart; blockIdx.z is this one
+  int px, py, pz;
+  long long bs;
+  // element offset from this box's fields to those of the box (sx, sy, sz) away, periodically
+  __device__ long long off(int sx, int sy, int sz) const {
+    const int b = (int)blockIdx.z;
+    const int x = (b % px + sx + px) % px, y = (b / px % py + sy + py) % py, z = (b / (px * py) + sz + pz) % pz;
+    return (long long)((z * py + y) * px + x - b) * bs;
+  }
+  template <typename T>
+  __device__ long long enter(T *&u, int sx, int sy, int sz) const {
+    u += (long long)blockIdx.z * bs;
+    return off(sx, sy, sz);
+  }
+};
 template <typename T>
-__global__ void k_ghost_z(T *base, size_t fs, int n, int g, long long lo, long long hi, T *dlt) {
+__global__ void k_ghost_z(T *base, size_t fs, int n, int g, ghost_boxes gb, T *dlt) {
   T *u = base + fs * blockIdx.y;
+  const long long lo = gb.enter(u, 0, 0, -1), hi = gb.off(0, 0, 1);
   const size_t n2 = (size_t)n * n;
   const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= (size_t)2 * g * n2) return;
@@ -107,8 +123,9 @@ __global__ void k_ghost_z(T *base, size_t fs, int n, int g, long long lo, long l
   u[(size_t)k * n2 + r] = v;
 }
 template <typename T>
-__global__ void k_ghost_y(T *base, size_t fs, int n, int g, long long lo, long long hi, T *dlt) {
+__global__ void k_ghost_y(T *base, size_t fs, int n, int g, ghost_boxes gb, T *dlt) {
   T *u = base + fs * blockIdx.y;
+  const long long lo = gb.enter(u, 0, -1, 0), hi = gb.off(0, 1, 0);
   const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int rows = 2 * g;
   if (t >= (size_t)(n - 2 * g) * rows * n) return;
@@ -122,8 +139,9 @@ __global__ void k_ghost_y(T *base, size_t fs, int n, int g, long long lo, long l
   u[IDX(n, k, j, i)] = v;
 }
 template <typename T>
-__global__ void k_ghost_x(T *base, size_t fs, int n, int g, long long lo, long long hi, T *dlt) {
+__global__ void k_ghost_x(T *base, size_t fs, int n, int g, ghost_boxes gb, T *dlt) {
   T *u = base + fs * blockIdx.y;
+  const long long lo = gb.enter(u, -1, 0, 0), hi = gb.off(1, 0, 0);
   const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int cols = 2 * g, m = n - 2 * g;
   if (t >= (size_t)m * m * cols) return;
@@ -229,13 +247,6 @@ __global__ __launch_bounds__(256) void k_ghost_fill(T *base, size_t fs, int n, i
   u[IDX(n, k, j, i)] = v;
 }
 
-// element offset from box b's fields to those of the box (sx, sy, sz) away
-static long long host_box_off(const etd_ctx *c, int b, int sx, int sy, int sz) {
-  const int bx = b % c->px, by = (b / c->px) % c->py, bz = b / (c->px * c->py);
-  const int x = (bx + sx + c->px) % c->px, y = (by + sy + c->py) % c->py, z = (bz + sz + c->pz) % c->pz;
-  return (long long)((z * c->py + y) * c->px + x - b) * (long long)c->bs;
-}
-
 // base: box 0's first field; the boxes' fields follow at stride bs.  dz, dy,
 // dx (one box only): record each sweep's changes (k_ghost_z/y/x)
 template <typename T>
@@ -257,15 +268,12 @@ void launch_ghost_fill(etd_ctx *c, T *base, int nfields, size_t fstride, T *dz, 
     etd_prof_end(c, PC_HALO);
     return;
   }
-  for (int b = 0; b < c->P; b++)
-    k_ghost_z<T><<<dim3((unsigned)((tz + 255) / 256), nfields), 256, 0, c->stream>>>(
-        base + b * c->bs, fstride, n, g, host_box_off(c, b, 0, 0, -1), host_box_off(c, b, 0, 0, 1), dz);
-  for (int b = 0; b < c->P; b++)
-    k_ghost_y<T><<<dim3((unsigned)((ty + 255) / 256), nfields), 256, 0, c->stream>>>(
-        base + b * c->bs, fstride, n, g, host_box_off(c, b, 0, -1, 0), host_box_off(c, b, 0, 1, 0), dy);
-  for (int b = 0; b < c->P; b++)
-    k_ghost_x<T><<<dim3((unsigned)((tx + 255) / 256), nfields), 256, 0, c->stream>>>(
-        base + b * c->bs, fstride, n, g, host_box_off(c, b, -1, 0, 0), host_box_off(c, b, 1, 0, 0), dx);
+  // one launch of each sweep for every box
+  const ghost_boxes gb = {c->px, c->py, c->pz, (long long)c->bs};
+  auto grid = [&](size_t t) { return dim3((unsigned)((t + 255) / 256), nfields, c->P); };
+  k_ghost_z<T><<<grid(tz), 256, 0, c->stream>>>(base, fstride, n, g, gb, dz);
+  k_ghost_y<T><<<grid(ty), 256, 0, c->stream>>>(base, fstride, n, g, gb, dy);
+  k_ghost_x<T><<<grid(tx), 256, 0, c->stream>>>(base, fstride, n, g, gb, dx);
   etd_prof_end(c, PC_HALO);
 }
 
@@ -768,11 +776,14 @@ void launch_modeprod(etd_ctx *c, const double *A4, const double *in, size_t in_f
 template <typename T>
 __global__ void k_phiscale(const T *uhat, const T *nhat, T *outp, size_t fs, int first_var, int nvars,
                            const double *DDX, const double *DDY, const double *DDZ, phi_args a, int order2,
-                           T *outp2) {
+                           T *outp2, size_t bs) {
   const int n = a.n;
   const size_t n3 = (size_t)n * n * n;
   const size_t l = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (l >= n3) return;
+  uhat += bs * blockIdx.y;  // a box of a decomposed run per blockIdx.y
+  nhat += bs * blockIdx.y;
+  outp += bs * blockIdx.y;
   int i, j, k;
   idx3(l, n, i, j, k);
   const int last = first_var + nvars;
@@ -816,13 +827,15 @@ __global__ void k_phiscale(const T *uhat, const T *nhat, T *outp, size_t fs, int
 }
 
 // out = (1 - phi1 H) uhat + phi1 nhat (or phi2 uhat), phi at the context's
-// current dt; out may be uhat
+// current dt; out may be uhat.  boxes: of a decomposed run, the given pointers
+// box 0's and the others' at stride bs
 template <typename T>
-void launch_phiscale(etd_ctx *c, const T *uhat, const T *nhat, T *out, int first_var, int nvars, int order2) {
+void launch_phiscale(etd_ctx *c, const T *uhat, const T *nhat, T *out, int first_var, int nvars, int order2,
+                     int boxes) {
   const phi_args a = phi_args_of(c, c->p.dt, 0.0);
   etd_prof_begin(c, PC_PHI);
-  k_phiscale<T><<<(unsigned)((c->n3 + 255) / 256), 256, 0, c->stream>>>(uhat, nhat, out, c->n3, first_var, nvars,
-                                                                      c->DDX, c->DDY, c->DDZ, a, order2, nullptr);
+  k_phiscale<T><<<dim3((unsigned)((c->n3 + 255) / 256), boxes), 256, 0, c->stream>>>(
+      uhat, nhat, out, c->n3, first_var, nvars, c->DDX, c->DDY, c->DDZ, a, order2, nullptr, c->bs);
   etd_prof_end(c, PC_PHI);
 }
 
@@ -835,7 +848,7 @@ void launch_phiscale_pair(etd_ctx *c, const T *uhat, const T *nhat, T *out, doub
   const phi_args a = phi_args_of(c, dt, dt2);
   etd_prof_begin(c, PC_PHI);
   k_phiscale<T><<<(unsigned)((c->n3 + 255) / 256), 256, 0, c->stream>>>(uhat, nhat, out, c->n3, first_var, nvars,
-                                                                      c->DDX, c->DDY, c->DDZ, a, 0, out2);
+                                                                      c->DDX, c->DDY, c->DDZ, a, 0, out2, 0);
   etd_prof_end(c, PC_PHI);
 }
 
@@ -846,6 +859,7 @@ struct nl_args {
   int slot0;        // Lbase mod ring
   double LE, KE, a2, a3, a4, epn2, hx, hy, hz, LCI, KCI, es;
   double ihx2, ihy2, ihz2;  // 1 / h^2, formed once on the host
+  double chx, chy, chz;     // 1 / 2h
   int phys;                 // physical boundaries on every side (periodic = 0, one box)
   int fe;                   // free energy: 0 Landau polynomial, 1 CALPHAD (alpha)
   double gbcc, ghcp;        // CALPHAD Gibbs energies (fe == 1)
@@ -870,6 +884,24 @@ __device__ __forceinline__ long long box_off(const nl_args &a, int sx, int sy, i
   y += y < 0 ? a.py : (y >= a.py ? -a.py : 0);
   z += z < 0 ? a.pz : (z >= a.pz ? -a.pz : 0);
   return (long long)((z * a.py + y) * a.px + x - ((a.bz * a.py + a.by) * a.px + a.bx)) * a.bs;
+}
+// a launch over every box of a decomposed run (one box per blockIdx.z): move
+// the fields, given for box 0, and the box's coordinates to this block's box
+template <typename T>
+__device__ __forceinline__ void enter_box(nl_args &a, const T *__restrict__ &u, T *__restrict__ &out,
+                                          const T *__restrict__ &sub) {
+  if (a.P == 1) return;
+  const int b = (int)blockIdx.z, m = a.n - 2 * a.g;
+  const long long o = b * a.bs;
+  u += o;
+  out += o;
+  if (sub) sub += o;
+  a.bx = b % a.px;
+  a.by = (b / a.px) % a.py;
+  a.bz = b / (a.px * a.py);
+  a.bxo = a.bx * m;
+  a.byo = a.by * m;
+  a.bzo = a.bz * m;
 }
 // The periodic interior image of extended position (z, y, x), -2 <= z, y, x
 // < n + 2, which the exchanged and relayed slabs hold (trans.c:7-925): in a
@@ -966,6 +998,7 @@ template <typename T, int FB>
 __global__ __launch_bounds__(256) void k_nonlin_ac(const T *__restrict__ u, T *__restrict__ out,
                                                    const T *__restrict__ sub, const T *__restrict__ E, nl_args a,
                                                    int with_felas, int mask_here) {
+  enter_box(a, u, out, sub);
   const int n = a.n, g = a.g;
   const unsigned n3 = (unsigned)n * n * n;  // n <= 272: every offset below fits 32 bits
   const size_t l = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1058,6 +1091,7 @@ template <typename T, int FB>
 __global__ __launch_bounds__(256) void k_nonlin_mix(const T *__restrict__ u, T *__restrict__ out,
                                                     const T *__restrict__ sub, const T *__restrict__ E, nl_args a,
                                                     int mask_here, const double *__restrict__ evs) {
+  enter_box(a, u, out, sub);
   const int n = a.n, g = a.g;
   const unsigned n3 = (unsigned)n * n * n;
   const size_t l = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1147,58 +1181,93 @@ __global__ __launch_bounds__(256) void k_nonlin_mix(const T *__restrict__ u, T *
   }(std::make_index_sequence<FB>{});
 }
 
-// ac_calc_F2 (anisotropic.c:164-627), pass 1: G = Lambda (gx, gy, gz) with
-// gy, gz taken as (u[-1] - u[+1]) / 2h; out-of-box neighbours read 0.
+// ac_calc_F2 (anisotropic.c:164-627): G = Lambda (gx, gy, gz) by central
+// differences, gy and gz taken as (u[-1] - u[+1]) / 2h; out -= epn2 LE div(G)
+// by the same differences (then the elastic term, keeping the reference's
+// order f1 - epn2 LE F2 - LE ES felas), every field and box in one launch.
+// Neighbours outside the box read 0, of u and of G; on a physical side the
+// low neighbour of cell 0 is the mirror cell 1.
+//
+// Both differences are formed from the 19 values of u that they need, with no
+// pass of G through memory (8 of the 11 passes that two launches per field
+// made): the six G at the neighbours share their twelve diagonal values, and
+// because a row of 68 cells leaves an end in nearly every wave, the ends are
+// clamped addresses and selects instead of branches.  Bound by the issue of
+// its 22 loads and some 300 instructions a point: 8 boxes x 4 fields of 68^3
+// FP64 337 -> 133 us (the bytes alone 60), 2 fields of 49^3 16 -> 8 us with
+// two launches instead of six.
 template <typename T>
-__global__ void k_f2_grad(const T *__restrict__ u, T *__restrict__ G, const double *__restrict__ lam, nl_args a) {
-  const int n = a.n;
+__global__ __launch_bounds__(256) void k_f2(const T *__restrict__ u, T *__restrict__ out, const T *__restrict__ sub,
+                                            const T *__restrict__ E, const double *__restrict__ lam, nl_args a,
+                                            int with_felas) {
+  enter_box(a, u, out, sub);
+  const int n = a.n, p = (int)blockIdx.y;
   const size_t n3 = (size_t)n * n * n;
   const size_t l = xcd_block() * blockDim.x + threadIdx.x;  // neighbours +-n, +-n^2 on this XCD
   if (l >= n3) return;
+  u += n3 * p;
+  out += n3 * p;
+  lam += 9 * p;
   int i, j, k;
   idx3(l, n, i, j, k);
-  // low neighbour of cell 0: 0 beside a neighbour, the mirror cell 1 on a physical side; high: 0
-  const double a_left = i > 0 ? u[l - 1] : (a.phys ? (double)u[l + 1] : 0.0);
-  const double a_right = i < n - 1 ? u[l + 1] : 0.0;
-  const double a_top = j > 0 ? u[l - n] : (a.phys ? (double)u[l + n] : 0.0);
-  const double a_bottom = j < n - 1 ? u[l + n] : 0.0;
-  const double a_front = k > 0 ? u[l - (size_t)n * n] : (a.phys ? (double)u[l + (size_t)n * n] : 0.0);
-  const double a_back = k < n - 1 ? u[l + (size_t)n * n] : 0.0;
-  const double gx = (a_right - a_left) / (2.0 * a.hx);
-  const double gy = (a_top - a_bottom) / (2.0 * a.hy);
-  const double gz = (a_front - a_back) / (2.0 * a.hz);
-  G[l] = (T)(lam[0] * gx + lam[1] * gy + lam[2] * gz);
-  G[n3 + l] = (T)(lam[3] * gx + lam[4] * gy + lam[5] * gz);
-  G[2 * n3 + l] = (T)(lam[6] * gx + lam[7] * gy + lam[8] * gz);
-}
-
-// pass 2: out -= epn2 LE div(G) (then the elastic term, keeping the
-// reference's order f1 - epn2 LE F2 - LE ES felas)
-template <typename T>
-__global__ void k_f2_div(const T *__restrict__ G, T *__restrict__ out, const T *__restrict__ E, nl_args a, int p,
-                         int with_felas, const T *__restrict__ u) {
-  const int n = a.n;
-  const size_t n3 = (size_t)n * n * n;
-  const size_t l = xcd_block() * blockDim.x + threadIdx.x;  // neighbours +-n, +-n^2 on this XCD
-  if (l >= n3) return;
-  int i, j, k;
-  idx3(l, n, i, j, k);
-  const T *gx = G, *gy = G + n3, *gz = G + 2 * n3;
-  const double a_left = i > 0 ? gx[l - 1] : (a.phys ? (double)gx[l + 1] : 0.0);
-  const double a_right = i < n - 1 ? gx[l + 1] : 0.0;
-  const double a_top = j > 0 ? gy[l - n] : (a.phys ? (double)gy[l + n] : 0.0);
-  const double a_bottom = j < n - 1 ? gy[l + n] : 0.0;
-  const double a_front = k > 0 ? gz[l - (size_t)n * n] : (a.phys ? (double)gz[l + (size_t)n * n] : 0.0);
-  const double a_back = k < n - 1 ? gz[l + (size_t)n * n] : 0.0;
-  double tmp = 0.0;
-  tmp += (a_right - a_left) / 2.0 / a.hx;
-  tmp += (a_top - a_bottom) / 2.0 / a.hy;
-  tmp += (a_front - a_back) / 2.0 / a.hz;
+  // bytes of a field fit 32 bits (n <= 272): one base plus a 32-bit offset
+  const int lo = (int)(l * sizeof(T)), sx = (int)sizeof(T), sy = n * sx, sz = n * sy;
+  auto at = [&](int off, bool in) {
+    const double v = (double)*(const T *)((const char *)u + (unsigned)(lo + off));
+    return in ? v : 0.0;
+  };
+  const double m = at(0, true);
+  // an axis: the offsets of its low and high neighbour and whether they count;
+  // u[high] - u[low] of the low and of the high neighbour cell
+  struct ax {
+    int off[2];
+    bool in[2];
+    double d[2];
+  };
+  auto axis = [&](int e, int st) {
+    ax r;
+    r.in[0] = e > 0 || a.phys;
+    r.in[1] = e < n - 1;
+    r.off[0] = e > 0 ? -st : a.phys ? st : 0;
+    r.off[1] = r.in[1] ? st : 0;
+    double up = m;  // the high neighbour of the low cell: this one, or cell 2 seen from the mirror cell 1
+    if (a.phys && e == 0) up = at(2 * st, true);
+    const double dn = at(e > 1 ? -2 * st : 0, e > 1 || a.phys);
+    const double far = at(e < n - 2 ? 2 * st : 0, e < n - 2);
+    r.d[0] = r.in[0] ? up - dn : 0.0;
+    r.d[1] = r.in[1] ? far - m : 0.0;
+    return r;
+  };
+  // what the field's own cell adds, asked for ahead of the stencil's arithmetic
   double f = out[l];
-  if (a.fe == 1 && with_felas) f -= a.LE * a.es * felas_at(E, a, p, k, j, i);  // the alpha driver's order
+  const double fe = with_felas ? felas_at(E, a, p, k, j, i) : 0.0, sb = sub ? (double)sub[n3 * p + l] : 0.0;
+  const ax X = axis(i, sx), Y = axis(j, sy), Z = axis(k, sz);
+  double xy[2][2], xz[2][2], yz[2][2];
+#pragma unroll
+  for (int s = 0; s < 2; s++)
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+      xy[s][t] = at(X.off[s] + Y.off[t], X.in[s] && Y.in[t]);
+      xz[s][t] = at(X.off[s] + Z.off[t], X.in[s] && Z.in[t]);
+      yz[s][t] = at(Y.off[s] + Z.off[t], Y.in[s] && Z.in[t]);
+    }
+  const double cx = a.chx, cy = a.chy, cz = a.chz;
+  double gx[2], gy[2], gz[2];  // component x of G at the two x neighbours, and so on
+#pragma unroll
+  for (int s = 0; s < 2; s++) {
+    gx[s] = lam[0] * (X.d[s] * cx) + lam[1] * ((xy[s][0] - xy[s][1]) * cy) + lam[2] * ((xz[s][0] - xz[s][1]) * cz);
+    gy[s] = lam[3] * ((xy[1][s] - xy[0][s]) * cx) + lam[4] * (-Y.d[s] * cy) + lam[5] * ((yz[s][0] - yz[s][1]) * cz);
+    gz[s] = lam[6] * ((xz[1][s] - xz[0][s]) * cx) + lam[7] * ((yz[0][s] - yz[1][s]) * cy) + lam[8] * (-Z.d[s] * cz);
+  }
+  double tmp = 0.0;
+  tmp += (gx[1] - gx[0]) * cx;
+  tmp += (gy[0] - gy[1]) * cy;
+  tmp += (gz[0] - gz[1]) * cz;
+  if (a.fe == 1 && with_felas) f -= a.LE * a.es * fe;  // the alpha driver's order
   f -= a.epn2 * a.LE * tmp;
-  if (a.fe != 1 && with_felas) f -= a.LE * a.es * felas_at(E, a, p, k, j, i);
-  if (a.mask && a.mask[l] == 0) f -= 0.5 * (double)u[l];
+  if (a.fe != 1 && with_felas) f -= a.LE * a.es * fe;
+  if (a.mask && a.mask[l] == 0) f -= 0.5 * m;
+  if (sub) f -= sb;
   out[l] = (T)f;
 }
 
@@ -1212,11 +1281,15 @@ __global__ void k_f2_div(const T *__restrict__ G, T *__restrict__ out, const T *
 template <typename T>
 __global__ __launch_bounds__(256) void k_f2_full(const T *__restrict__ u, T *__restrict__ out,
                                                  const T *__restrict__ sub, const T *__restrict__ E,
-                                                 const double *__restrict__ lam, nl_args a, int p, int with_felas) {
-  const int n = a.n;
+                                                 const double *__restrict__ lam, nl_args a, int with_felas) {
+  enter_box(a, u, out, sub);
+  const int n = a.n, p = (int)blockIdx.y;
   const size_t n3 = (size_t)n * n * n;
   const size_t l = xcd_block() * blockDim.x + threadIdx.x;
   if (l >= n3) return;
+  u += n3 * p;
+  out += n3 * p;
+  lam += 9 * p;
   int i, j, k;
   idx3(l, n, i, j, k);
   const bool inner = i > 0 && i < n - 1 && j > 0 && j < n - 1 && k > 0 && k < n - 1;
@@ -1255,7 +1328,7 @@ __global__ __launch_bounds__(256) void k_f2_full(const T *__restrict__ u, T *__r
   f -= a.epn2 * a.LE * t;
   if (a.fe != 1 && with_felas) f -= a.LE * a.es * felas_at(E, a, p, k, j, i);
   if (a.mask && a.mask[l] == 0) f -= 0.5 * (double)u[l];
-  if (sub) f -= (double)sub[l];
+  if (sub) f -= (double)sub[n3 * p + l];
   out[l] = (T)f;
 }
 
@@ -1355,6 +1428,7 @@ template <typename T>
 __global__ __launch_bounds__(256) void k_ch_nl(const T *__restrict__ c, T *__restrict__ out, const T *__restrict__ sub,
                                                const float *__restrict__ nc, const T *__restrict__ E, int q, nl_args a,
                                                unsigned nbi8) {
+  enter_box(a, c, out, sub);
   const int n = a.n;
   const ch_h ih = {a.ihx2, a.ihy2, a.ihz2};
   const unsigned b = blockIdx.x;
@@ -1418,16 +1492,6 @@ __global__ __launch_bounds__(256) void k_ch_nl(const T *__restrict__ c, T *__res
   out[l] = (T)r;
 }
 
-template <typename T>
-__global__ void k_sub(T *out, const T *sub, size_t cnt) {
-  const size_t l = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (l < cnt) out[l] = out[l] - sub[l];
-}
-template <typename T>
-void launch_sub(etd_ctx *c, T *out, const T *sub, size_t cnt) {
-  k_sub<T><<<(unsigned)((cnt + 255) / 256), 256, 0, c->stream>>>(out, sub, cnt);
-}
-
 static nl_args make_nl(etd_ctx *c) {
   nl_args a;
   a.n = c->n;
@@ -1455,6 +1519,9 @@ static nl_args make_nl(etd_ctx *c) {
   a.ihx2 = 1.0 / (a.hx * a.hx);
   a.ihy2 = 1.0 / (a.hy * a.hy);
   a.ihz2 = 1.0 / (a.hz * a.hz);
+  a.chx = 0.5 / a.hx;
+  a.chy = 0.5 / a.hy;
+  a.chz = 0.5 / a.hz;
   a.phys = !c->p.periodic;
   a.fe = c->p.free_energy;
   a.gbcc = c->gbcc;
@@ -1636,12 +1703,15 @@ static void launch_ch_nl(etd_ctx *c, const T *cf, T *out, const T *sub, const fl
   const long NI = c->n - 4;
   const unsigned nbi8 = round8((size_t)((NI * NI * NI + 255) / 256));
   const unsigned nbs = (unsigned)((shell_count(c->n) + 255) / 256);
-  k_ch_nl<T><<<nbi8 + nbs, 256, 0, c->stream>>>(cf, out, sub, nc, fields<T>(c).E, q, a, nbi8);
+  k_ch_nl<T><<<dim3(nbi8 + nbs, 1, c->P), 256, 0, c->stream>>>(cf, out, sub, nc, fields<T>(c).E, q, a, nbi8);
 }
 
-// N for every variable into out (V x n3); when sub != NULL the result is
-// N - sub (the ETD2 difference prepare_U1_new, calc.c:537-551).  ch_centre
-// (mixed path): the CH outputs are N - N(c_mean), the centred term.
+// N for every variable of every box into out (V x n3; out, sub: box 0's first
+// field, the others at stride bs); each box reads its neighbours' fields for
+// the outside values, so all boxes are evaluated before any is advanced.  When
+// sub != NULL the result is N - sub (the ETD2 difference prepare_U1_new,
+// calc.c:537-551).  ch_centre (mixed path): the CH outputs are N - N(c_mean),
+// the centred term.
 template <typename T>
 void launch_nonlinear(etd_ctx *c, T *out, const T *sub, int ch_centre) {
   nl_args a = make_nl(c);
@@ -1649,6 +1719,7 @@ void launch_nonlinear(etd_ctx *c, T *out, const T *sub, int ch_centre) {
   const size_t n3 = c->n3;
   const unsigned nb = (unsigned)((n3 + 255) / 256);
   const int felas = c->p.elastic == 1 && c->nac > 0;
+  const unsigned P = (unsigned)c->P;
   etd_prof_begin(c, PC_NONLIN);
   if (c->nac > 0) {
     const int aniso = c->p.anisotropic;
@@ -1664,30 +1735,24 @@ void launch_nonlinear(etd_ctx *c, T *out, const T *sub, int ch_centre) {
     const int mh = aniso ? 0 : 1;  // the grain mask goes with the last pass over the field
     if (felas && c->el_mix) {
       if (c->nac <= 8)
-        k_nonlin_mix<T, 8><<<nb, 256, 0, c->stream>>>(F.u, out, sb, F.E, a, mh, a.ev);
+        k_nonlin_mix<T, 8><<<dim3(nb, 1, P), 256, 0, c->stream>>>(F.u, out, sb, F.E, a, mh, a.ev);
       else if (c->nac <= 12)
-        k_nonlin_mix<T, 12><<<nb, 256, 0, c->stream>>>(F.u, out, sb, F.E, a, mh, a.ev);
+        k_nonlin_mix<T, 12><<<dim3(nb, 1, P), 256, 0, c->stream>>>(F.u, out, sb, F.E, a, mh, a.ev);
       else
-        k_nonlin_mix<T, 16><<<nb, 256, 0, c->stream>>>(F.u, out, sb, F.E, a, mh, a.ev);
+        k_nonlin_mix<T, 16><<<dim3(nb, 1, P), 256, 0, c->stream>>>(F.u, out, sb, F.E, a, mh, a.ev);
     } else if (fb == 4)
-      k_nonlin_ac<T, 4><<<nb, 256, 0, c->stream>>>(F.u, out, sb, F.E, a, fl, mh);
+      k_nonlin_ac<T, 4><<<dim3(nb, 1, P), 256, 0, c->stream>>>(F.u, out, sb, F.E, a, fl, mh);
     else if (fb == 8)
-      k_nonlin_ac<T, 8><<<nb, 256, 0, c->stream>>>(F.u, out, sb, F.E, a, fl, mh);
+      k_nonlin_ac<T, 8><<<dim3(nb, 1, P), 256, 0, c->stream>>>(F.u, out, sb, F.E, a, fl, mh);
     else if (fb == 12)
-      k_nonlin_ac<T, 12><<<nb, 256, 0, c->stream>>>(F.u, out, sb, F.E, a, fl, mh);
+      k_nonlin_ac<T, 12><<<dim3(nb, 1, P), 256, 0, c->stream>>>(F.u, out, sb, F.E, a, fl, mh);
     else
-      k_nonlin_ac<T, 16><<<nb, 256, 0, c->stream>>>(F.u, out, sb, F.E, a, fl, mh);
+      k_nonlin_ac<T, 16><<<dim3(nb, 1, P), 256, 0, c->stream>>>(F.u, out, sb, F.E, a, fl, mh);
     const int felas2 = felas && !c->el_mix;
-    if (aniso == 1)
-      for (int p = 0; p < c->nac; p++) {
-        k_f2_grad<T><<<round8(nb), 256, 0, c->stream>>>(F.u + n3 * p, F.gtmp, c->lam + 9 * p, a);
-        k_f2_div<T><<<round8(nb), 256, 0, c->stream>>>(F.gtmp, out + n3 * p, F.E, a, p, felas2, F.u + n3 * p);
-        if (sub) launch_sub(c, out + n3 * p, sub + n3 * p, n3);  // after the F2 / felas terms
-      }
-    if (aniso == 2)
-      for (int p = 0; p < c->nac; p++)
-        k_f2_full<T><<<round8(nb), 256, 0, c->stream>>>(F.u + n3 * p, out + n3 * p, sub ? sub + n3 * p : nullptr,
-                                                        F.E, c->lam + 9 * p, a, p, felas2);
+    // every field and box in one launch, and N(u) of every box above
+    const dim3 grid(round8(nb), c->nac, P);
+    if (aniso == 1) k_f2<T><<<grid, 256, 0, c->stream>>>(F.u, out, sub, F.E, c->lam, a, felas2);
+    if (aniso == 2) k_f2_full<T><<<grid, 256, 0, c->stream>>>(F.u, out, sub, F.E, c->lam, a, felas2);
   }
   if (c->p.variable_mobility)
     launch_vm<T>(c, F.u, out, sub, F.gtmp, a);
@@ -2946,7 +3011,7 @@ void ch_mean_restore(etd_ctx *c, float *u) {
 
 #define ETD_INST(T)                                                                   \
   template void launch_ghost_fill<T>(etd_ctx *, T *, int, size_t, T *, T *, T *);    \
-  template void launch_phiscale<T>(etd_ctx *, const T *, const T *, T *, int, int, int); \
+  template void launch_phiscale<T>(etd_ctx *, const T *, const T *, T *, int, int, int, int); \
   template void launch_phiscale_pair<T>(etd_ctx *, const T *, const T *, T *, double, T *, double, int, int); \
   template void launch_nonlinear<T>(etd_ctx *, T *, const T *, int);                 \
   template void launch_elastic<T>(etd_ctx *);                                        \
