@@ -1391,10 +1391,10 @@ __device__ double ch_mu_out(const T *c, const T *E, int q, const nl_args &a, con
 // Points whose whole stencil is at least one cell from the box faces (the
 // inner (n - 4)^3) need t only pointwise; the others (the shell, two cells
 // thick) need the face terms, the outside values and mu_out.  The grid keeps
-// them apart so every wave runs one of the two paths: blocks [0, nbi8) take
-// the inner points (x fastest, blocks spread over the XCDs in contiguous
-// ranges so the +-n^2 neighbours share an L2), the rest the shell points in
-// the order of shell_point.
+// them apart so every wave runs one of the two paths: blocks [0, nbs8) take
+// the shell points in the order of shell_point (the longer waves first), the
+// other nbi8 the inner points (x fastest, blocks spread over the XCDs in
+// contiguous ranges so the +-n^2 neighbours share an L2).
 __device__ __forceinline__ void shell_point(long s, int n, int &i, int &j, int &k) {
   const long n2 = (long)n * n, ring = 8L * n - 16;  // points of a middle plane's shell
   if (s < 4 * n2) {                                   // planes 0, 1, n - 2, n - 1
@@ -1425,14 +1425,14 @@ __host__ __device__ __forceinline__ long shell_count(int n) {
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void k_ch_nl(const T *__restrict__ c, T *__restrict__ out, const T *__restrict__ sub,
+__global__ __launch_bounds__(256, 7) void k_ch_nl(const T *__restrict__ c, T *__restrict__ out, const T *__restrict__ sub,
                                                const float *__restrict__ nc, const T *__restrict__ E, int q, nl_args a,
-                                               unsigned nbi8) {
+                                               unsigned nbs8, unsigned nbi8) {
   enter_box(a, c, out, sub);
   const int n = a.n;
   const ch_h ih = {a.ihx2, a.ihy2, a.ihz2};
-  const unsigned b = blockIdx.x;
-  if (b < nbi8) {
+  if (blockIdx.x >= nbs8) {
+    const unsigned b = blockIdx.x - nbs8;
     const int NI = n - 4;
     const size_t bb = (size_t)(b & 7u) * (nbi8 >> 3) + (b >> 3);
     const size_t li = bb * blockDim.x + threadIdx.x;
@@ -1459,19 +1459,67 @@ __global__ __launch_bounds__(256) void k_ch_nl(const T *__restrict__ c, T *__res
     out[l] = (T)r;
     return;
   }
-  const long s = (long)(b - nbi8) * blockDim.x + threadIdx.x;
+  const long s = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= shell_count(n)) return;
   int i, j, k;
   shell_point(s, n, i, j, k);
   const size_t l = IDX(n, k, j, i);
-  const double tc = ch_t_at(c, E, q, a, ih, k, j, i);
-  const double f_right = i < n - 1 ? ch_t_at(c, E, q, a, ih, k, j, i + 1) : 0.0;
-  const double f_bottom = j < n - 1 ? ch_t_at(c, E, q, a, ih, k, j + 1, i) : 0.0;
-  const double f_back = k < n - 1 ? ch_t_at(c, E, q, a, ih, k + 1, j, i) : 0.0;
+  // t at the cell and those of its six neighbours that the box has (as
+  // ch_t_at).  A wave here has cells of every kind, so a load of its own
+  // behind each condition was a chain of some fifty latencies: the seven values, and
+  // per axis that has a face here the seven image values, are asked for
+  // together (the empty statements keep the compiler from moving them behind
+  // the selects).  FP64 n = 49 15.8 -> 8.5 us, FP32 n = 104 20.9 -> 12.4, n =
+  // 196 60.5 -> 58.8 (there the inner points' HBM counts; 8 waves per SIMD)
+  const long long st[3] = {(long long)n * n, n, 1};
+  const int e[3] = {k, j, i};
+  bool has[7];
+  double t[7], w[7];
+  int pz[7], py[7], px[7];
+#pragma unroll
+  for (int m = 0; m < 7; m++) {
+    const int ax = m == 0 ? 0 : (m - 1) / 2, d = m == 0 ? 0 : m & 1 ? -1 : 1, x = e[ax] + d;
+    has[m] = x >= 0 && x < n;
+    const int dd = has[m] ? d : 0;
+    pz[m] = k + (ax == 0 ? dd : 0);
+    py[m] = j + (ax == 1 ? dd : 0);
+    px[m] = i + (ax == 2 ? dd : 0);
+    t[m] = c[(long long)l + dd * st[ax]];
+  }
+  asm volatile("" : "+v"(t[0]), "+v"(t[1]), "+v"(t[2]), "+v"(t[3]), "+v"(t[4]), "+v"(t[5]), "+v"(t[6]));
+#pragma unroll
+  for (int m = 0; m < 7; m++) {
+    const double cc = t[m];
+    double f = -a.LCI * a.KCI * cc;
+    f += a.LCI * ch_f(cc);
+    if (a.elastic == 2) f += a.LCI * felas_at(E, a, q, pz[m], py[m], px[m]);
+    t[m] = f;
+  }
+  if (!a.phys) {  // outside values
+    const double ce = a.LCI * a.epn2;
+#pragma unroll
+    for (int ax = 2; ax >= 0; ax--) {  // x, y, z
+      if (e[ax] > 1 && e[ax] < n - 2) continue;  // none of the seven lies on a face of this axis
+      const double h2 = ax == 2 ? ih.x : ax == 1 ? ih.y : ih.z;
+      bool face[7];
+#pragma unroll
+      for (int m = 0; m < 7; m++) {
+        const int x = ax == 2 ? px[m] : ax == 1 ? py[m] : pz[m];
+        face[m] = x == 0 || x == n - 1;
+        const int o = face[m] ? x == 0 ? -1 : n : x;
+        const int z = ax == 0 ? o : pz[m], y = ax == 1 ? o : py[m], xx = ax == 2 ? o : px[m];
+        w[m] = Pimg(c, a, z, y, xx);
+      }
+      asm volatile("" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]), "+v"(w[4]), "+v"(w[5]), "+v"(w[6]));
+#pragma unroll
+      for (int m = 0; m < 7; m++) t[m] = face[m] ? t[m] - ce * w[m] * h2 : t[m];
+    }
+  }
+  const double tc = t[0], f_back = has[2] ? t[2] : 0.0, f_bottom = has[4] ? t[4] : 0.0, f_right = has[6] ? t[6] : 0.0;
   // low neighbour of cell 0: 0 beside a neighbour, the mirror (cell 1) on a physical side
-  const double f_left = i > 0 ? ch_t_at(c, E, q, a, ih, k, j, i - 1) : (a.phys ? f_right : 0.0);
-  const double f_top = j > 0 ? ch_t_at(c, E, q, a, ih, k, j - 1, i) : (a.phys ? f_bottom : 0.0);
-  const double f_front = k > 0 ? ch_t_at(c, E, q, a, ih, k - 1, j, i) : (a.phys ? f_back : 0.0);
+  const double f_front = has[1] ? t[1] : (a.phys ? f_back : 0.0);
+  const double f_top = has[3] ? t[3] : (a.phys ? f_bottom : 0.0);
+  const double f_left = has[5] ? t[5] : (a.phys ? f_right : 0.0);
   double r = (f_left + f_right - 2.0 * tc) * ih.x;
   r += (f_top + f_bottom - 2.0 * tc) * ih.y;
   r += (f_front + f_back - 2.0 * tc) * ih.z;
@@ -1481,12 +1529,9 @@ __global__ __launch_bounds__(256) void k_ch_nl(const T *__restrict__ c, T *__res
     out[l] = (T)r;
     return;
   }
-  if (i == 0) r -= ch_mu_out(c, E, q, a, ih, k, j, -1) * ih.x;
-  if (i == n - 1) r -= ch_mu_out(c, E, q, a, ih, k, j, n) * ih.x;
-  if (j == 0) r -= ch_mu_out(c, E, q, a, ih, k, -1, i) * ih.y;
-  if (j == n - 1) r -= ch_mu_out(c, E, q, a, ih, k, n, i) * ih.y;
-  if (k == 0) r -= ch_mu_out(c, E, q, a, ih, -1, j, i) * ih.z;
-  if (k == n - 1) r -= ch_mu_out(c, E, q, a, ih, n, j, i) * ih.z;
+  if (i == 0 || i == n - 1) r -= ch_mu_out(c, E, q, a, ih, k, j, i == 0 ? -1 : n) * ih.x;
+  if (j == 0 || j == n - 1) r -= ch_mu_out(c, E, q, a, ih, k, j == 0 ? -1 : n, i) * ih.y;
+  if (k == 0 || k == n - 1) r -= ch_mu_out(c, E, q, a, ih, k == 0 ? -1 : n, j, i) * ih.z;
   if (sub) r -= sub[l];
   if (nc) r -= nc[l];
   out[l] = (T)r;
@@ -1702,8 +1747,8 @@ template <typename T>
 static void launch_ch_nl(etd_ctx *c, const T *cf, T *out, const T *sub, const float *nc, int q, const nl_args &a) {
   const long NI = c->n - 4;
   const unsigned nbi8 = round8((size_t)((NI * NI * NI + 255) / 256));
-  const unsigned nbs = (unsigned)((shell_count(c->n) + 255) / 256);
-  k_ch_nl<T><<<dim3(nbi8 + nbs, 1, c->P), 256, 0, c->stream>>>(cf, out, sub, nc, fields<T>(c).E, q, a, nbi8);
+  const unsigned nbs8 = round8((size_t)((shell_count(c->n) + 255) / 256));
+  k_ch_nl<T><<<dim3(nbs8 + nbi8, 1, c->P), 256, 0, c->stream>>>(cf, out, sub, nc, fields<T>(c).E, q, a, nbs8, nbi8);
 }
 
 // N for every variable of every box into out (V x n3; out, sub: box 0's first
