@@ -4,8 +4,13 @@
 // A copy to or from pageable memory goes through the runtime's pinned buffer
 // on one thread: 17 GB/s for the 60 MB of an FP64 field at n = 196, and for
 // FP32 storage a second pass on that thread converts, into pages that are
-// fresh each time.  Here a field passes through three pinned slots: the calling thread keeps the copies going, up to HC_THREADS
-// others convert (or copy) their share of each chunk that has arrived.
+// fresh each time.  Here a field passes through three pinned slots: the
+// calling thread keeps the copies going, and it and up to HC_THREADS - 1
+// others convert (or copy) pieces of the chunks that have arrived.
+// A piece goes to whoever is free and nobody waits for a thread that has not
+// begun: after a caller's OpenMP region its threads hold every CPU for a
+// while, a new thread then starts 3 to 4 ms late, and the calling thread does
+// the work alone.
 // Measured, one field read (set), before against now: n = 196 FP64 3.4 (2.0)
 // -> 1.4 (1.4) ms, FP32 3.5 (2.7) -> 0.8 (0.8) ms; n = 260 FP32 21.8 (16.3)
 // -> 1.6 (1.7) ms; n = 36 FP32 21 to 90 -> 20 us.  Chunks: a copy costs about 13 us
@@ -14,11 +19,13 @@
 #include <hip/hip_runtime.h>
 #include <emmintrin.h>
 #include <pthread.h>
+#include <sched.h>
 #include <stdlib.h>
 #include <string.h>
 
 #include <atomic>
 #include <mutex>
+#include <new>
 #include <utility>
 
 #include "etd_internal.h"
@@ -27,6 +34,7 @@
 #define HC_CHUNK ((size_t)4 << 20)   // most device bytes per slot
 #define HC_SHARE ((size_t)8 << 20)   // host bytes that pay for one more thread (from two on)
 #define HC_SLOTS 3
+#define HC_PIECES 8                  // of a chunk, for the threads
 #define HC_MIN ((size_t)64 << 10)    // least device bytes per slot
 // FP64 fields up to this: the runtime's own path (n = 68, read 147 us there,
 // 142 here, set 100 and 128; n = 84 read 273 and 222, set 148 and 190; n = 100
@@ -70,11 +78,11 @@ struct hc_job {
   size_t cnt, per;  // elements in all, per chunk
   size_t nch;       // chunks
   int put;
-  // the workers' side: chunks they may take, chunks each has finished
-  int nt;
-  std::atomic<size_t> ready;
-  std::atomic<size_t> done[HC_THREADS];
-  std::atomic<int> stop;
+  // the host side: pieces of the chunks below ready go to whoever takes the
+  // next one; done counts the finished ones of each slot
+  size_t pc;   // elements per piece, HC_PIECES of them per chunk
+  std::atomic<size_t> ready, next, done[HC_SLOTS];
+  std::atomic<int> refs;  // who still looks at this record
 
   void *pin;        // HC_SLOTS chunks
 
@@ -95,49 +103,63 @@ struct hc_job {
 };
 
 template <typename T>
-struct hc_arg {
-  hc_job<T> *j;
-  int t;
-};
+static bool hc_take(hc_job<T> *j) {
+  size_t i = j->next.load(std::memory_order_relaxed);
+  do {
+    if (i >= j->ready.load(std::memory_order_acquire) * HC_PIECES) return false;
+  } while (!j->next.compare_exchange_weak(i, i + 1, std::memory_order_relaxed));
+  const size_t k = i / HC_PIECES, n = j->len(k), a = i % HC_PIECES * j->pc, b = a + j->pc < n ? a + j->pc : n;
+  if (b > a) j->part(k, a, b);
+  j->done[k % HC_SLOTS].fetch_add(1, std::memory_order_release);
+  return true;
+}
+// workers that run or are yet to, of all calls: no more than HC_LIVE are made
+#define HC_LIVE 12
+static std::atomic<int> hc_live;
 
-// a worker converts (or copies) its share of every chunk; it makes no HIP
-// call (a thread's first one costs a few hundred microseconds)
+template <typename T>
+static void hc_drop(hc_job<T> *j) {
+  if (j->refs.fetch_sub(1, std::memory_order_acq_rel) == 1) delete j;
+}
+// a worker makes no HIP call (a thread's first one costs a few hundred
+// microseconds); one that comes after the last piece finds nothing to take
 template <typename T>
 static void *hc_thread(void *p) {
-  hc_job<T> *j = ((hc_arg<T> *)p)->j;
-  const int t = ((hc_arg<T> *)p)->t;
-  for (size_t k = 0; k < j->nch; k++) {
-    while (j->ready.load(std::memory_order_acquire) <= k) {
-      if (j->stop.load(std::memory_order_relaxed)) return nullptr;
-      _mm_pause();
-    }
-    // shares in whole cache lines of the host buffer
-    const size_t n = j->len(k), nt = j->nt, sh = ((n + nt - 1) / nt + 7) & ~(size_t)7;
-    const size_t a = t * sh < n ? t * sh : n, b = a + sh < n ? a + sh : n;
-    if (b > a) j->part(k, a, b);
-    j->done[t].store(k + 1, std::memory_order_release);
-  }
+  hc_job<T> *j = (hc_job<T> *)p;
+  while (j->next.load(std::memory_order_relaxed) < j->nch * HC_PIECES)
+    if (!hc_take(j)) _mm_pause();
+  hc_drop(j);
+  hc_live.fetch_sub(1, std::memory_order_release);
   return nullptr;
 }
+template <typename T>
+static bool hc_worker(hc_job<T> *j) {
+  if (hc_live.fetch_add(1, std::memory_order_relaxed) < HC_LIVE) {
+    pthread_t th;
+    j->refs.fetch_add(1, std::memory_order_relaxed);
+    if (!pthread_create(&th, nullptr, hc_thread<T>, j)) {
+      (void)pthread_detach(th);
+      return true;
+    }
+    j->refs.fetch_sub(1, std::memory_order_relaxed);
+  }
+  hc_live.fetch_sub(1, std::memory_order_relaxed);
+  return false;
+}
 
-// the calling thread: copies and events, and the conversion itself when
-// there are no workers
+// the calling thread: copies and events, and pieces while it waits for them
 template <typename T>
 static hipError_t hc_run(hc_job<T> *j) {
   hipError_t e = hipSuccess;
-  auto finish = [&](size_t k) {  // the host side of chunk k
-    if (j->nt == 0) return j->part(k, 0, j->len(k));
-    j->ready.store(k + 1, std::memory_order_release);
-  };
   auto finished = [&](size_t k) {
-    for (int t = 0; t < j->nt; t++)
-      while (j->done[t].load(std::memory_order_acquire) <= k) _mm_pause();
+    while (j->done[k % HC_SLOTS].load(std::memory_order_acquire) < (k / HC_SLOTS + 1) * HC_PIECES)
+      if (!hc_take(j)) _mm_pause();
   };
   if (j->put) {
     for (size_t k = 0; k <= j->nch; k++) {
       if (k < j->nch) {
         if (k >= HC_SLOTS && (e = j->wait(k - HC_SLOTS)) != hipSuccess) return e;
-        finish(k);
+        j->ready.store(k + 1, std::memory_order_release);
       }
       if (k == 0) continue;
       finished(k - 1);
@@ -149,7 +171,7 @@ static hipError_t hc_run(hc_job<T> *j) {
     if ((e = j->start(k)) != hipSuccess) return e;
   for (size_t k = 0; k < j->nch; k++) {
     if ((e = j->wait(k)) != hipSuccess) return e;
-    finish(k);
+    j->ready.store(k + 1, std::memory_order_release);
     if (k == 0 || k - 1 + HC_SLOTS >= j->nch) continue;
     finished(k - 1);
     if ((e = j->start(k - 1 + HC_SLOTS)) != hipSuccess) return e;
@@ -214,8 +236,10 @@ void host_copy_open(void) {
 void host_copy_close(etd_ctx *c) {
   for (int i = 0; i < c->io_nev; i++) (void)hipEventDestroy(c->io_ev[i]);
   std::lock_guard<std::mutex> l(pool_mu);
-  if (--pool_users == 0)
+  if (--pool_users == 0) {
+    while (hc_live.load(std::memory_order_acquire)) sched_yield();  // late workers: the library may be unloaded next
     while (pool_n) (void)hipHostFree(pool_buf[--pool_n].p);
+  }
 }
 
 // the slots' events; 0 when they cannot be had
@@ -267,30 +291,36 @@ hipError_t host_copy(etd_ctx *c, T *dev, double *host, size_t cnt, int put) {
   size_t pinned = 0;
   void *pin = hc_events(c) ? pool_take((nch < HC_SLOTS ? nch : HC_SLOTS) * per, &pinned) : nullptr;
   if (!pin) return hc_one(c, dev, host, cnt, put);
-  hc_job<T> job;
-  job.pin = pin;
-  job.c = c;
-  job.dev = dev;
-  job.host = host;
-  job.cnt = cnt;
-  job.per = per / sizeof(T);
-  job.nch = nch;
-  job.put = put;
-  job.ready = 0;
-  job.stop = 0;
-  hc_arg<T> arg[HC_THREADS];
-  pthread_t th[HC_THREADS];
-  int want = (int)(sizeof(double) * cnt / HC_SHARE), made = 0;
-  want = want < 2 ? 0 : want > HC_THREADS ? HC_THREADS : want;
-  for (; made < want; made++) {
-    job.done[made] = 0;
-    arg[made] = hc_arg<T>{&job, made};
-    if (pthread_create(&th[made], nullptr, hc_thread<T>, &arg[made])) break;  // fewer threads, or none, do as well
+  hc_job<T> *const j = new (std::nothrow) hc_job<T>;
+  if (!j) {
+    pool_give(pin, pinned);
+    return hc_one(c, dev, host, cnt, put);
   }
-  job.nt = made;  // read by a worker after its first chunk is ready
-  hipError_t e = hc_run(&job);
-  job.stop = 1;
-  for (int t = 0; t < made; t++) (void)pthread_join(th[t], nullptr);
+  j->pin = pin;
+  j->c = c;
+  j->dev = dev;
+  j->host = host;
+  j->cnt = cnt;
+  j->per = per / sizeof(T);
+  j->nch = nch;
+  j->put = put;
+  j->pc = (j->per / HC_PIECES + 8) & ~(size_t)7;  // whole cache lines of the host buffer
+  j->ready = 0;
+  j->next = 0;
+  for (int t = 0; t < HC_SLOTS; t++) j->done[t] = 0;
+  j->refs = 1;
+  int want = (int)(sizeof(double) * cnt / HC_SHARE) - 1;  // the calling thread is one
+  want = want > HC_THREADS - 1 ? HC_THREADS - 1 : want;
+  while (want > 0 && hc_worker(j)) want--;  // fewer threads, or none, do as well
+  hipError_t e = hc_run(j);
+  // no piece is given out any more (after an error some are left); those that
+  // were are done before the buffers are anyone else's
+  size_t taken = j->next.exchange(nch * HC_PIECES), got;
+  do {
+    got = 0;
+    for (int t = 0; t < HC_SLOTS; t++) got += j->done[t].load(std::memory_order_acquire);
+  } while (got < taken);
+  hc_drop(j);
   // the slots are free, and what was put is on the device, after this
   const hipError_t es = hipStreamSynchronize(c->stream);
   pool_give(pin, pinned);
