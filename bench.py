@@ -297,16 +297,16 @@ def main():
         # field passes the mode products made (3 axes x the fields of each
         # transform: 2V forward and V backward, or nch + V forward when the
         # AC spectrum is carried), counted by the library
-        mp_flops = ms[9] * 2.0 * n ** 4
+        mp_flops = ms[9] * 1.0 * n ** 4  # done: the basis' parity halves the 2 n^4 of a field pass
         mp_launch_ms = ms[1] / max(1, launches[0])
         fp = {"sim_time_per_s": dt * K / (ms[0] / 1e3), "steps": K, "warmup": Wm, "ms_per_step": ms[0] / K,
               "grid_point_variant_steps_per_s": N ** 3 * V * K / (ms[0] / 1e3), "breakdown_ms_per_step": breakdown(ms, K),
-              "roofline": {"kernel": "k_modeprod_dl<13,4,2,2> (FP64 MFMA 4x4x4 mode products)", "bound": "mfma",
+              "roofline": {"kernel": "k_modeprod_fold<13> (FP64 MFMA 4x4x4 mode products, folded by parity)", "bound": "mfma",
                            "achieved": mp_flops / (ms[1] / 1e3) / 1e12, "peak": PEAK_FP64_MFMA / 1e12,
                            "unit": "TFLOP/s", "frac": mp_flops / (ms[1] / 1e3) / PEAK_FP64_MFMA,
                            "field_passes_per_step": ms[9] / K,
                            "launch_ms_avg": mp_launch_ms, "launches": launches[0],
-                           "traffic": traffic_per_launch("k_modeprod_dl_192cube_13fields_hbm_counters.md",
+                           "traffic": traffic_per_launch("k_modeprod_fold_192cube_hbm_counters.md",
                                                          ms[9] / max(1, launches[0]))}}
 
     # ---- mixed precision, fixed dt: per-kernel timing of the headline path's kernels
@@ -318,17 +318,19 @@ def main():
         mx = {"ms_per_step": ms[0] / K, "sim_time_per_s_fixed_dt": dt * K / (ms[0] / 1e3),
               "grid_point_variant_steps_per_s": N ** 3 * V * K / (ms[0] / 1e3), "breakdown_ms_per_step": breakdown(ms, K)}
         fft_launch_ms = ms[7] / max(1, launches[6]) / 3.0  # 3 axis passes per fft3d group
-        npair = (nac + 1) // 2
-        fft_bytes = 2 * npair * N ** 3 * 8.0  # read + write one float2 per point and packed field
+        # packed fields of a pass: pairs of variants, or (more than six) of the six strain components, which the
+        # first pass forms from all the fields; read + write one float2 per point, the average of the six passes
+        npair = 3 if nac > 6 else (nac + 1) // 2
+        fft_bytes = (11 * npair * 8.0 + nac * 4.0) / 6.0 * N ** 3
         mp_launch_ms = ms[1] / max(1, launches[0])
         mp_fields_avg = ms[9] / max(1, launches[0])  # fields per launch (a launch is one axis pass)
         mp_bytes = 2 * 4.0 * n ** 3 * mp_fields_avg  # read + write FP32 per field
         nterm = 6 if args.precision == 1 else 3  # BF16 split-3: six products; FP16 split-2: three
         mp_mfma = nterm * 2.0 * n ** 4 * mp_fields_avg
-        r_fft = {"kernel": "k_fft16<12> (own two-stage register FFT pass, FP32 in HBM)", "bound": "hbm",
+        r_fft = {"kernel": "k_fft2<16,12> (own two-stage register FFT pass, FP32 in HBM)", "bound": "hbm",
                  "achieved": fft_bytes / (fft_launch_ms / 1e3) / 1e9, "peak": PEAK_HBM / 1e9, "unit": "GB/s",
                  "frac": fft_bytes / (fft_launch_ms / 1e3) / PEAK_HBM,
-                 "traffic": measured_traffic("k_fft16_f32_192cube_hbm_counters.md"), "launch_ms": fft_launch_ms,
+                 "traffic": measured_traffic("k_fft2_f32_192cube_hbm_counters.md"), "launch_ms": fft_launch_ms,
                  "ms_per_step": ms[7] / K}
         r_mp = {"kernel": ("k_modeprod_split_p (split-BF16 x3 MFMA, FP32 accumulate)" if args.precision == 1 else
                            "k_modeprod_f16_r3<13,2> (split-FP16 x2 MFMA, contraction over the slowest axis, "

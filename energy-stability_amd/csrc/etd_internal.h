@@ -291,7 +291,7 @@ template <typename T>
 int launch_diag(etd_ctx *c, double *stats);
 /* doubles of partial sums one check_soln_new evaluation writes (the size of c->part) */
 size_t etd_diag_partials(const etd_ctx *c);
-/* the two-stage register FFT (k_fft16) handles this N */
+/* the two-stage register FFT (k_fft2) handles this N */
 bool fft16_supported(int N);  /* N = 16 R2 */
 bool fft2_supported(int N);   /* any two-stage transform (etd_fft2.hip) */
 /* CH mean conservation of the mixed path: ch_mean_mark takes the interior

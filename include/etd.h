@@ -389,7 +389,7 @@ typedef struct etd_tuning {
   int mp_variant;      /* FP64 mode products: 0, 1, 2 (direct-to-LDS), 4 (register-staged), 16 (16x16x4);
                           1 (the default) takes half-size products where V and V^-1 have parity */
   int split_waves;     /* mixed mode products: 8 or 4 waves per workgroup (0: by size) */
-  int fft_variant;     /* 1: two-stage register FFT (16 | N), 0: radix passes */
+  int fft_variant;     /* 1: two-stage register FFT where N has an instance, 0: radix passes */
   double ms_per_step;  /* measured by etd_autotune */
 } etd_tuning;
 /* Times `steps` fixed-dt steps of every candidate on a scratch context with
