@@ -47,9 +47,8 @@ struct etd_dev_consts {
   double C4[81];
   double sig[ETD_MAX_VAR * 9];
   double t0[ETD_MAX_VAR * ETD_MAX_VAR];
-  /* with el_mix: the six components of every variant's eigenstrain (xx, yy,
-   * zz, yz, xz, xy of its symmetric part); sig and t0 are then those of the
-   * six unit strains */
+  /* with el_mix: every variant's components of the six strains that are
+   * transformed (strain_basis); sig and t0 are then those strains' */
   double ev[ETD_MAX_VAR * 6];
 };
 

@@ -2122,7 +2122,13 @@ __device__ __forceinline__ void b_wrow(const double *sp, const double *nv, const
 // with a = acc_2r, b = acc_2r+1.
 // Arithmetic in the storage precision: FP64 for FP64 fields, FP32 for the
 // mixed path's FP32 spectra (half the registers: 4 waves per SIMD instead of
-// 2 at NAC = 12); the geometry Omega(n) is always formed in FP64.
+// 2 at NAC = 12); the geometry Omega(n) is always formed in FP64.  With six
+// fields B is too: it is a difference of terms some five times its size, and
+// six strains in place of more variants add roundings of their own.  The mixed
+// force of 7 to 16 variants is then 0.16 to 0.63 times as far from the FP64
+// one as a transform per variant with FP32 B was (n = 36 .. 196, volume to
+// shear strains); a step's elasticity, N = 192 626 -> 632 us, four waves per
+// SIMD as before (with FP64 in the mirror points, few, one).
 template <int NAC, bool MIRROR, typename T2, bool WRITE_NEG = false>
 __device__ __forceinline__ void contract_point(const T2 *__restrict__ Z, T2 *__restrict__ Y, int N,
                                                int npair, size_t m, const etd_dev_consts *__restrict__ K) {
@@ -2144,42 +2150,43 @@ __device__ __forceinline__ void contract_point(const T2 *__restrict__ Z, T2 *__r
     F[2 * r] = C2{(CT)0.5 * (a.x + b.x), (CT)0.5 * (a.y - b.y)};
     if (2 * r + 1 < NAC) F[2 * r + 1] = C2{(CT)0.5 * (a.y + b.y), (CT)-0.5 * (a.x - b.x)};
   }
-  CT nv[3], om[9];
+  using BT = typename std::conditional<NAC == 6 && !MIRROR, double, CT>::type;
+  BT nv[3], om[9];
   {
     double nvd[3], omd[9];
     b_geometry(signed_wave(x, N), signed_wave(y, N), signed_wave(z, N), K, nvd, omd);
 #pragma unroll
-    for (int k = 0; k < 3; k++) nv[k] = (CT)nvd[k];
+    for (int k = 0; k < 3; k++) nv[k] = (BT)nvd[k];
 #pragma unroll
-    for (int k = 0; k < 9; k++) om[k] = (CT)omd[k];
+    for (int k = 0; k < 9; k++) om[k] = (BT)omd[k];
   }
   // b_q = sigma_q n for every variant; c_p = b_p Omega only for the row p
   // being summed (3 live values instead of 3 NAC: fewer VGPRs, more waves)
-  CT bv[NAC][3];
+  BT bv[NAC][3];
 #pragma unroll
   for (int q = 0; q < NAC; q++) {
     const double *sg = K->sig + 9 * q;
 #pragma unroll
     for (int k = 0; k < 3; k++)
-      bv[q][k] = (CT)sg[k * 3 + 0] * nv[0] + (CT)sg[k * 3 + 1] * nv[1] + (CT)sg[k * 3 + 2] * nv[2];
+      bv[q][k] = (BT)sg[k * 3 + 0] * nv[0] + (BT)sg[k * 3 + 1] * nv[1] + (BT)sg[k * 3 + 2] * nv[2];
   }
-  CT bm[MIRROR ? NAC : 1][3], cm[MIRROR ? NAC : 1][3];
+  BT bm[MIRROR ? NAC : 1][3], cm[MIRROR ? NAC : 1][3];
   if constexpr (MIRROR) {
-    CT nv2[3], om2[9];
+    BT nv2[3], om2[9];
     {
       double nvd[3], omd[9];
       b_geometry(signed_wave(xm, N), signed_wave(ym, N), signed_wave(zm, N), K, nvd, omd);
 #pragma unroll
-      for (int k = 0; k < 3; k++) nv2[k] = (CT)nvd[k];
+      for (int k = 0; k < 3; k++) nv2[k] = (BT)nvd[k];
 #pragma unroll
-      for (int k = 0; k < 9; k++) om2[k] = (CT)omd[k];
+      for (int k = 0; k < 9; k++) om2[k] = (BT)omd[k];
     }
 #pragma unroll
     for (int q = 0; q < NAC; q++) {
       const double *sg = K->sig + 9 * q;
 #pragma unroll
       for (int k = 0; k < 3; k++)
-        bm[q][k] = (CT)sg[k * 3 + 0] * nv2[0] + (CT)sg[k * 3 + 1] * nv2[1] + (CT)sg[k * 3 + 2] * nv2[2];
+        bm[q][k] = (BT)sg[k * 3 + 0] * nv2[0] + (BT)sg[k * 3 + 1] * nv2[1] + (BT)sg[k * 3 + 2] * nv2[2];
 #pragma unroll
       for (int k = 0; k < 3; k++)
         cm[q][k] = bm[q][0] * om2[0 * 3 + k] + bm[q][1] * om2[1 * 3 + k] + bm[q][2] * om2[2 * 3 + k];
@@ -2190,15 +2197,16 @@ __device__ __forceinline__ void contract_point(const T2 *__restrict__ Z, T2 *__r
   for (int p = 0; p < NAC; p++) acc[p] = C2{(CT)0, (CT)0};
 #pragma unroll
   for (int p = 0; p < NAC; p++) {
-    CT cvp[3];
+    BT cvp[3];
 #pragma unroll
     for (int k = 0; k < 3; k++) cvp[k] = bv[p][0] * om[0 * 3 + k] + bv[p][1] * om[1 * 3 + k] + bv[p][2] * om[2 * 3 + k];
 #pragma unroll
     for (int q = p; q < NAC; q++) {
-      const CT t0 = (CT)K->t0[p * ETD_MAX_VAR + q];
-      CT B = t0 - (cvp[0] * bv[q][0] + cvp[1] * bv[q][1] + cvp[2] * bv[q][2]);
+      const BT t0 = (BT)K->t0[p * ETD_MAX_VAR + q];
+      BT Bd = t0 - (cvp[0] * bv[q][0] + cvp[1] * bv[q][1] + cvp[2] * bv[q][2]);
       if constexpr (MIRROR)
-        B = (CT)0.5 * (B + (t0 - (cm[p][0] * bm[q][0] + cm[p][1] * bm[q][1] + cm[p][2] * bm[q][2])));
+        Bd = (BT)0.5 * (Bd + (t0 - (cm[p][0] * bm[q][0] + cm[p][1] * bm[q][1] + cm[p][2] * bm[q][2])));
+      const CT B = (CT)Bd;
       acc[p].x += F[q].x * B;
       acc[p].y += F[q].y * B;
       if (q != p) {
@@ -2344,7 +2352,7 @@ __global__ void k_el_unpack_mix(const typename cplx<T>::t *__restrict__ Y, T *__
 // B_pq is bilinear in the variants' eigenstrains, B_pq = sum_ab ev_pa B_ab
 // ev_qb over the six components of a symmetric strain, so with more than six
 // variants (el_mix) the six fields g_a = sum_q ev_qa eta_q are transformed,
-// contracted with the B of the six unit strains and transformed back, and
+// contracted with the B of the six strains (strain_basis) and transformed back, and
 // felas_p = sum_a ev_pa G_a is formed where it is used: 3 packed transforms
 // each way instead of 6 for 12 variants, and 6 fields to read in the
 // nonlinear term instead of 12.  Up to six variants it saves nothing.
