@@ -216,7 +216,12 @@ __global__ __launch_bounds__(256) void k_ghost_fill(T *base, size_t fs, int n, i
       if (dlt) dlt[fd + rec] = (T)((double)v - (double)u[to]);
       u[to] = v;
     };
-    // every lane's reads of the two rows come before any lane's writes: one wave runs in step
+    // Every lane's reads of the two rows come before any lane's writes, also
+    // of the x ghosts that another lane holds in a[]: the fence keeps the
+    // compiler from moving a read past a write, and a wave's memory operations
+    // go in order.  It adds no instruction.
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int c = 0; c < 5; c++) {
       const int i = lane + 64 * c;
