@@ -242,14 +242,19 @@ void host_copy_close(etd_ctx *c) {
   }
 }
 
-// the slots' events; 0 when they cannot be had
+// the slots' events; 0 when they cannot be had.  An event belongs to the
+// device that is current when it is made, and the calling thread may have
+// another one than the context's.
 static int hc_events(etd_ctx *c) {
-  for (; c->io_nev < HC_SLOTS; c->io_nev++)
-    if (hipEventCreateWithFlags(&c->io_ev[c->io_nev], hipEventDisableTiming) != hipSuccess) {
-      (void)hipGetLastError();
-      return 0;
-    }
-  return 1;
+  if (c->io_nev == HC_SLOTS) return 1;
+  int cur = c->device;
+  hipError_t e = hipGetDevice(&cur);
+  if (e == hipSuccess && cur != c->device) e = hipSetDevice(c->device);
+  for (; e == hipSuccess && c->io_nev < HC_SLOTS; c->io_nev += e == hipSuccess)
+    e = hipEventCreateWithFlags(&c->io_ev[c->io_nev], hipEventDisableTiming);
+  if (cur != c->device) (void)hipSetDevice(cur);
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e == hipSuccess;
 }
 
 // one copy: FP64 directly, FP32 through one slot, or the heap where pinned

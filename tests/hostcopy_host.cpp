@@ -1,0 +1,146 @@
+// The field copies (csrc/etd_hostcopy.hip) on the CPU: the source itself with
+// the few HIP calls that it makes replaced by a model of the runtime.  Device
+// memory is host memory; copies and events run only when something waits for
+// them, in stream order, so a slot that is read or reused too early shows.
+// An event must be of the device of the stream that it is recorded on.
+#include <stdio.h>
+#include <string.h>
+
+#include <deque>
+#include <map>
+#include <random>
+#include <string>
+#include <vector>
+
+#include "etd_hostcopy.hip"
+
+static int cur_dev;
+struct op {
+  void *to;
+  const void *from;
+  size_t bytes;
+  hipEvent_t ev;
+};
+static std::deque<op> queue;          // of the one stream
+static const int stream_dev = 1;
+static std::map<hipEvent_t, int> event_dev;
+static int copies, mallocs;
+static const void *copied_host;       // the host side of the last copy
+
+static void run_until(hipEvent_t ev) {
+  while (!queue.empty()) {
+    const op o = queue.front();
+    queue.pop_front();
+    if (o.bytes) memcpy(o.to, o.from, o.bytes);
+    if (ev && o.ev == ev) return;
+  }
+}
+hipError_t hipGetDevice(int *d) {
+  *d = cur_dev;
+  return hipSuccess;
+}
+hipError_t hipSetDevice(int d) {
+  cur_dev = d;
+  return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void *to, const void *from, size_t bytes, hipMemcpyKind kind, hipStream_t) {
+  queue.push_back({to, from, bytes, nullptr});
+  copies++;
+  copied_host = kind == hipMemcpyHostToDevice ? from : to;
+  return hipSuccess;
+}
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) {
+  *e = (hipEvent_t) new int;
+  event_dev[*e] = cur_dev;
+  return hipSuccess;
+}
+hipError_t hipEventDestroy(hipEvent_t e) {
+  event_dev.erase(e);
+  delete (int *)e;
+  return hipSuccess;
+}
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t) {
+  if (event_dev.at(e) != stream_dev) return hipErrorInvalidHandle;
+  queue.push_back({nullptr, nullptr, 0, e});
+  return hipSuccess;
+}
+hipError_t hipEventSynchronize(hipEvent_t e) {
+  run_until(e);
+  return hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t) {
+  run_until(nullptr);
+  return hipSuccess;
+}
+hipError_t hipHostMalloc(void **p, size_t bytes, unsigned) {
+  mallocs++;
+  *p = malloc(bytes);
+  return *p ? hipSuccess : hipErrorOutOfMemory;
+}
+hipError_t hipHostFree(void *p) {
+  free(p);
+  return hipSuccess;
+}
+hipError_t hipGetLastError(void) { return hipSuccess; }
+
+#define CHECK(x)                                       \
+  do {                                                 \
+    if (!(x)) {                                        \
+      printf("line %d: %s\n", __LINE__, #x);           \
+      exit(1);                                         \
+    }                                                  \
+  } while (0)
+
+struct context {
+  etd_ctx c = {};
+  explicit context(int dev = stream_dev) {
+    c.device = stream_dev;
+    cur_dev = dev;
+    host_copy_open();
+  }
+  ~context() { host_copy_close(&c); }
+};
+
+template <typename T>
+static void trip(context &x, size_t cnt, size_t offset) {
+  std::mt19937_64 r(cnt + offset);
+  std::vector<char> a(8 * cnt + 64), b(8 * cnt + 64);
+  std::vector<T> dev(cnt);
+  double *from = (double *)(a.data() + offset), *to = (double *)(b.data() + offset);
+  for (size_t i = 0; i < cnt; i++) {
+    const double v = (double)(int64_t)r() * 0x1p-40;
+    memcpy(from + i, &v, 8);
+  }
+  CHECK(host_copy<T>(&x.c, dev.data(), from, cnt, 1) == hipSuccess && queue.empty());
+  CHECK(host_copy<T>(&x.c, dev.data(), to, cnt, 0) == hipSuccess && queue.empty());
+  for (size_t i = 0; i < cnt; i++) {
+    double u, v;
+    memcpy(&u, from + i, 8);
+    memcpy(&v, to + i, 8);
+    CHECK((double)(T)u == v);
+  }
+}
+// fields of n^3: one copy, two chunks, four chunks and more, none to three helper threads, a short last chunk
+static void trips() {
+  context x;
+  for (size_t n : {1, 12, 68, 84, 104, 132, 148, 164, 197}) {
+    trip<double>(x, n * n * n, 0);
+    trip<float>(x, n * n * n, 8);
+  }
+  trip<float>(x, 84 * 84 * 84, 0);
+}
+// the calling thread's device is another than the context's
+static void device() {
+  context x(0);
+  trip<double>(x, 148 * 148 * 148, 0);
+  trip<float>(x, 148 * 148 * 148, 0);
+  CHECK(cur_dev == 0);
+}
+
+int main(int, char **argv) {
+  const std::map<std::string, void (*)()> what = {{"trips", trips}, {"device", device}};
+  what.at(argv[1])();
+  CHECK(event_dev.empty());
+  puts("ok");
+  return 0;
+}
