@@ -20,6 +20,7 @@
 #include <emmintrin.h>
 #include <pthread.h>
 #include <sched.h>
+#include <signal.h>
 #include <stdlib.h>
 #include <string.h>
 
@@ -327,7 +328,14 @@ hipError_t host_copy(etd_ctx *c, T *dev, double *host, size_t cnt, int put) {
   j->refs = 1;
   int want = (int)(sizeof(double) * cnt / HC_SHARE) - 1;  // the calling thread is one
   want = want > HC_THREADS - 1 ? HC_THREADS - 1 : want;
-  while (want > 0 && hc_worker(j)) want--;  // fewer threads, or none, do as well
+  if (want > 0) {
+    // the process's signals stay with its own threads: a helper inherits a mask that blocks them all
+    sigset_t all, old;
+    sigfillset(&all);
+    const int masked = !pthread_sigmask(SIG_SETMASK, &all, &old);
+    while (want > 0 && masked && hc_worker(j)) want--;  // fewer threads, or none, do as well
+    if (masked) (void)pthread_sigmask(SIG_SETMASK, &old, nullptr);
+  }
   hipError_t e = hc_run(j);
   // no piece is given out any more (after an error some are left); those that
   // were are done before the buffers are anyone else's

@@ -12,7 +12,14 @@
 #include <string>
 #include <vector>
 
+#include <signal.h>
+
+// the thread calls of the copies are looked at on the way
+static int model_create(pthread_t *, const pthread_attr_t *, void *(*)(void *), void *);
+#include <pthread.h>
+#define pthread_create model_create
 #include "etd_hostcopy.hip"
+#undef pthread_create
 
 static int cur_dev;
 struct op {
@@ -91,6 +98,24 @@ hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *p) {
 }
 hipError_t hipGetLastError(void) { return hipSuccess; }
 
+static std::atomic<int> made, unblocked;  // helper threads, and those that a signal could run on
+struct entry {
+  void *(*f)(void *);
+  void *arg;
+};
+static void *enter(void *p) {
+  const entry e = *(entry *)p;
+  delete (entry *)p;
+  sigset_t now;
+  pthread_sigmask(SIG_SETMASK, nullptr, &now);
+  if (!sigismember(&now, SIGINT) || !sigismember(&now, SIGALRM) || !sigismember(&now, SIGUSR1)) unblocked++;
+  return e.f(e.arg);
+}
+static int model_create(pthread_t *t, const pthread_attr_t *a, void *(*f)(void *), void *arg) {
+  made++;
+  return pthread_create(t, a, enter, new entry{f, arg});
+}
+
 #define CHECK(x)                                       \
   do {                                                 \
     if (!(x)) {                                        \
@@ -160,11 +185,23 @@ static void pinned() {
       CHECK(copies > 2);
     }
 }
+// the process's signals stay with its own threads
+static void signals() {
+  context x;
+  sigset_t before, after;
+  pthread_sigmask(SIG_SETMASK, nullptr, &before);
+  trip<double>(x, 164 * 164 * 164, 0);
+  trip<float>(x, 164 * 164 * 164, 0);
+  pthread_sigmask(SIG_SETMASK, nullptr, &after);
+  CHECK(made > 0 && sigismember(&after, SIGINT) == sigismember(&before, SIGINT));
+}
 
 int main(int, char **argv) {
-  const std::map<std::string, void (*)()> what = {{"trips", trips}, {"device", device}, {"pinned", pinned}};
+  const std::map<std::string, void (*)()> what = {{"trips", trips}, {"device", device}, {"pinned", pinned},
+                                                     {"signals", signals}};
   what.at(argv[1])();
   CHECK(event_dev.empty());
+  CHECK(argv[1] != std::string("signals") || unblocked == 0);
   puts("ok");
   return 0;
 }
