@@ -19,7 +19,6 @@
 #include <hip/hip_runtime.h>
 #include <emmintrin.h>
 #include <pthread.h>
-#include <sched.h>
 #include <signal.h>
 #include <stdlib.h>
 #include <string.h>
@@ -114,9 +113,19 @@ static bool hc_take(hc_job<T> *j) {
   j->done[k % HC_SLOTS].fetch_add(1, std::memory_order_release);
   return true;
 }
-// workers that run or are yet to, of all calls: no more than HC_LIVE are made
+// the helper threads of all calls, HC_LIVE at most (four copies at a time get
+// all three of theirs, later ones do with fewer).  A place is taken by one call (HC_CLAIMED), its
+// thread made and finished; then the next call that takes it, or the last
+// context to close, joins the thread: the library may be unloaded after that.
 #define HC_LIVE 12
-static std::atomic<int> hc_live;
+#define HC_MADE 1
+#define HC_FINISHED 2
+#define HC_CLAIMED 4
+static struct hc_place {
+  pthread_t th;
+  std::atomic<int> st;
+  void *job;
+} hc_at[HC_LIVE];
 
 template <typename T>
 static void hc_drop(hc_job<T> *j) {
@@ -126,25 +135,29 @@ static void hc_drop(hc_job<T> *j) {
 // microseconds); one that comes after the last piece finds nothing to take
 template <typename T>
 static void *hc_thread(void *p) {
-  hc_job<T> *j = (hc_job<T> *)p;
+  hc_place *const at = (hc_place *)p;
+  hc_job<T> *j = (hc_job<T> *)at->job;
   while (j->next.load(std::memory_order_relaxed) < j->nch * HC_PIECES)
     if (!hc_take(j)) _mm_pause();
   hc_drop(j);
-  hc_live.fetch_sub(1, std::memory_order_release);
+  at->st.fetch_or(HC_FINISHED, std::memory_order_release);
   return nullptr;
 }
 template <typename T>
 static bool hc_worker(hc_job<T> *j) {
-  if (hc_live.fetch_add(1, std::memory_order_relaxed) < HC_LIVE) {
-    pthread_t th;
+  for (hc_place &at : hc_at) {
+    int st = at.st.load(std::memory_order_acquire);
+    if ((st != 0 && st != (HC_MADE | HC_FINISHED)) ||
+        !at.st.compare_exchange_strong(st, HC_CLAIMED, std::memory_order_acquire))
+      continue;
+    if (st) (void)pthread_join(at.th, nullptr);
+    at.job = j;
     j->refs.fetch_add(1, std::memory_order_relaxed);
-    if (!pthread_create(&th, nullptr, hc_thread<T>, j)) {
-      (void)pthread_detach(th);
-      return true;
-    }
-    j->refs.fetch_sub(1, std::memory_order_relaxed);
+    const bool ok = !pthread_create(&at.th, nullptr, hc_thread<T>, &at);
+    if (!ok) j->refs.fetch_sub(1, std::memory_order_relaxed);
+    at.st.fetch_xor(ok ? HC_CLAIMED | HC_MADE : HC_CLAIMED, std::memory_order_release);
+    return ok;
   }
-  hc_live.fetch_sub(1, std::memory_order_relaxed);
   return false;
 }
 
@@ -238,7 +251,11 @@ void host_copy_close(etd_ctx *c) {
   for (int i = 0; i < c->io_nev; i++) (void)hipEventDestroy(c->io_ev[i]);
   std::lock_guard<std::mutex> l(pool_mu);
   if (--pool_users == 0) {
-    while (hc_live.load(std::memory_order_acquire)) sched_yield();  // late workers: the library may be unloaded next
+    for (hc_place &at : hc_at)
+      if (at.st.load(std::memory_order_acquire) & HC_MADE) {
+        (void)pthread_join(at.th, nullptr);
+        at.st.store(0, std::memory_order_relaxed);
+      }
     while (pool_n) (void)hipHostFree(pool_buf[--pool_n].p);
   }
 }

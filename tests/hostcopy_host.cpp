@@ -10,6 +10,7 @@
 #include <map>
 #include <random>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include <signal.h>
@@ -17,9 +18,12 @@
 // the thread calls of the copies are looked at on the way
 static int model_create(pthread_t *, const pthread_attr_t *, void *(*)(void *), void *);
 #include <pthread.h>
+static int model_join(pthread_t, void **);
 #define pthread_create model_create
+#define pthread_join model_join
 #include "etd_hostcopy.hip"
 #undef pthread_create
+#undef pthread_join
 
 static int cur_dev;
 struct op {
@@ -98,7 +102,8 @@ hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *p) {
 }
 hipError_t hipGetLastError(void) { return hipSuccess; }
 
-static std::atomic<int> made, unblocked;  // helper threads, and those that a signal could run on
+// helper threads: made, joined, and those that a signal could run on
+static std::atomic<int> made, joined, unblocked;
 struct entry {
   void *(*f)(void *);
   void *arg;
@@ -114,6 +119,10 @@ static void *enter(void *p) {
 static int model_create(pthread_t *t, const pthread_attr_t *a, void *(*f)(void *), void *arg) {
   made++;
   return pthread_create(t, a, enter, new entry{f, arg});
+}
+static int model_join(pthread_t t, void **r) {
+  joined++;
+  return pthread_join(t, r);
 }
 
 #define CHECK(x)                                       \
@@ -195,12 +204,37 @@ static void signals() {
   pthread_sigmask(SIG_SETMASK, nullptr, &after);
   CHECK(made > 0 && sigismember(&after, SIGINT) == sigismember(&before, SIGINT));
 }
+// no helper is left, not even in its last instructions, when the last context
+// has closed: the library may be unloaded then.  Several threads copy at once.
+static void threads() {
+  context x;
+  std::vector<std::thread> th;
+  for (int t = 0; t < 4; t++)
+    th.emplace_back([t] {
+      for (int k = 0; k < 3; k++) {
+        std::vector<float> buf(148 * 148 * 148);
+        hc_job<float> *j = new hc_job<float>;
+        j->c = nullptr, j->dev = nullptr, j->host = nullptr, j->put = 0;
+        j->cnt = buf.size(), j->per = buf.size(), j->nch = 1, j->pc = buf.size() / HC_PIECES, j->pin = buf.data();
+        std::vector<double> out(buf.size());
+        j->host = out.data();
+        j->ready = 1, j->next = 0, j->refs = 1;
+        for (auto &d : j->done) d = 0;
+        for (int w = 0; w < 3; w++) hc_worker(j);
+        while (hc_take(j)) {}
+        while (j->done[0] < HC_PIECES) _mm_pause();
+        hc_drop(j);
+      }
+    });
+  for (auto &t : th) t.join();
+}
 
 int main(int, char **argv) {
   const std::map<std::string, void (*)()> what = {{"trips", trips}, {"device", device}, {"pinned", pinned},
-                                                     {"signals", signals}};
+                                                     {"signals", signals}, {"threads", threads}};
   what.at(argv[1])();
   CHECK(event_dev.empty());
+  CHECK(argv[1] != std::string("threads") || (made > 3 && joined == made));
   CHECK(argv[1] != std::string("signals") || unblocked == 0);
   puts("ok");
   return 0;

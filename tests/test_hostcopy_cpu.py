@@ -19,10 +19,10 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("what", ["trips", "device", "pinned", "signals"])
+@pytest.mark.parametrize("what", ["trips", "device", "pinned", "signals", "threads"])
 def test_copies(program, what):
     """trips: what comes back is what was set, over every way a copy goes; device: from a thread whose current
     device is not the context's; pinned: a buffer that the runtime knows is copied in one piece;
-    signals: the helper threads block them."""
+    signals: the helper threads block them; threads: all of them are joined once the last context is closed."""
     r = subprocess.run([program, what], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and r.stdout.endswith("ok\n"), r.stdout + r.stderr
