@@ -318,13 +318,8 @@ template <int RT, bool EVEN, bool FWD>
 static void fold_go(etd_ctx *c, const double *Af, const double *in, size_t in_fs, double *out, size_t out_fs,
                     int nfields, int e0, int accumulate) {
   using CF = fold_cfg<RT>;
-  static_assert(2 * CF::LDS <= 160 * 1024, "two workgroups per CU");
-  static bool attr_set = false;
-  if (!attr_set) {
-    (void)hipFuncSetAttribute((const void *)k_modeprod_fold<RT, EVEN, FWD>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, CF::LDS);
-    attr_set = true;
-  }
+  // two workgroups per CU, and what a launch may ask for without an attribute set on every device first
+  static_assert(2 * CF::LDS <= 160 * 1024 && CF::LDS <= 64 * 1024, "LDS");
   const dim3 grid((unsigned)((c->n * c->n + FOLD_COLS - 1) / FOLD_COLS), nfields);
   k_modeprod_fold<RT, EVEN, FWD><<<grid, 256, CF::LDS, c->stream>>>(Af, in, in_fs, out, out_fs, c->n, e0, accumulate);
 }
