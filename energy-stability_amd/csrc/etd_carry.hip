@@ -200,20 +200,36 @@ static size_t carry_elems(const etd_ctx *c, size_t *off) {
 // Whether carrying pays.  It saves three field passes of the mode products
 // per AC field and costs the correction: two batched GEMMs, the axis factors
 // and a pass whose blocks are few and long on small boxes (19 us at n = 36).
-// FP64, fixed ETD1 steps without elasticity, carried against transforming u:
-// n = 36 x 4 fields 70 / 47 us, 68 x 4 112 / 89, 100 x 4 198 / 194, 116 x 4
-// 282 / 289, 84 x 12 367 / 358, 100 x 12 561 / 572, 132 x 1 178 / 171,
-// 164 x 1 249 / 283, 196 x 12 4152 / 5032: the line lies near n^3 sqrt(nac) =
-// 2.7e6.  ETD2 corrects twice a step: 132 x 12 2520 / 2365, 164 x 12 4854 /
-// 4881, 196 x 4 2764 / 2767, 260 x 4 6792 / 7178.  With physical sides there
-// are no GEMMs: 68 x 4 81 / 82, ETD2 68 x 4 164 / 155, 100 x 4 317 / 341.
+// FP64, fixed ETD1 steps without elasticity, carried against transforming u by
+// folded products: n = 36 x 4 fields 70 / 47 us, 68 x 4 112 / 89, 100 x 4 198 /
+// 194, 116 x 4 282 / 289, 84 x 12 367 / 358, 100 x 12 561 / 572, 132 x 1 178 /
+// 171, 164 x 1 249 / 283, 196 x 12 4152 / 5032: the line lies near n^3
+// sqrt(nac) = 2.7e6.  ETD2 corrects twice a step: 132 x 12 2520 / 2365, 164 x
+// 12 4854 / 4881, 196 x 4 2764 / 2767, 260 x 4 6792 / 7178.  With physical
+// sides there are no GEMMs: 68 x 4 81 / 82, ETD2 68 x 4 164 / 155, 100 x 4 317 /
+// 341.
+// Full-size products (a basis without parity, as those read from files, or
+// another variant chosen) make what is saved dearer: 76 x 4 134 / 118, 92 x 4
+// 205 / 208, 116 x 1 156 / 152, 132 x 1 231 / 251, 76 x 12 335 / 320, 92 x 12
+// 513 / 552; the odd edges, whose full product is the slow one, 45 x 12 172 /
+// 158, 85 x 1 218 / 183, 85 x 4 248 / 285; ETD2 116 x 4 782 / 759, 132 x 4
+// 1198 / 1206, 100 x 12 1413 / 1383, 116 x 12 2221 / 2251, 164 x 12 6782 /
+// 7253; physical sides 60 x 4 68 / 68, 68 x 4 93 / 102, 52 x 12 110 / 126, ETD2
+// 76 x 4 203 / 203, 92 x 1 177 / 174, 100 x 1 207 / 212.
 // The mixed path carries at any size: it is the more accurate of the two
-// there (u is not rounded by a transform of its own every step).
+// there (u is not rounded by a transform of its own every step).  In FP64 it
+// is too, within rounding: after 20 steps at n = 68 1.5e-15 from the exact
+// sequence carried, 8.8e-15 transformed (1.1e-14 by full products).
 static bool carry_pays(const etd_ctx *c) {
   if (c->mixed || c->carry_always) return true;
   const double m = (double)c->n3 * sqrt((double)c->nac);
-  if (!c->p.periodic) return m >= (c->p.etd2 ? 1.5e6 : 0.6e6);
-  return m >= (c->p.etd2 ? 15e6 : 2.7e6);
+  const bool etd2 = c->p.etd2;
+  if (c->mp_variant == 1 && c->Vf) {
+    if (!c->p.periodic) return m >= (etd2 ? 1.5e6 : 0.6e6);
+    return m >= (etd2 ? 15e6 : 2.7e6);
+  }
+  if (!c->p.periodic) return m >= (etd2 ? 0.8e6 : 0.45e6);
+  return m >= (etd2 ? 4.5e6 : c->n % 2 ? 1.0e6 : 1.5e6);
 }
 
 // one box, two ghost layers, a size at which it pays, and coefficients whose exp(-dt H) factors stay
