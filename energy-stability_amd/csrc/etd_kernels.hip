@@ -2407,14 +2407,14 @@ void launch_elastic(etd_ctx *c) {
     const unsigned nbh = (unsigned)(((size_t)N * N * (N / 2 + 1) + 255) / 256);
     const T2 *Zc = (const T2 *)F.Z;
     T2 *Yc = (T2 *)F.Y;
-    bool one = false;
+    constexpr int ONE_MAX = sizeof(T) == 4 ? 6 : 5;  // the joint kernel's registers
+    const bool one = c->nft <= ONE_MAX && (sizeof(T) == 4 || N <= 168);
     switch (c->nft) {
 #define NACC(X)                                                                                       \
   case X:                                                                                             \
-    if constexpr (X <= (sizeof(T) == 4 ? 6 : 5)) one = sizeof(T) == 4 || N <= 168;                    \
     if (one) {                                                                                        \
-      if constexpr (X <= 6)                                                                           \
-      k_el_contract_one<X, T2><<<nbm + nbh, 256, 0, c->stream>>>(Zc, Yc, N, c->npair, c->dconst, nbm); \
+      if constexpr (X <= ONE_MAX)                                                                     \
+        k_el_contract_one<X, T2><<<nbm + nbh, 256, 0, c->stream>>>(Zc, Yc, N, c->npair, c->dconst, nbm); \
     } else {                                                                                          \
       k_el_contract_t<X, T2><<<nbh, 256, 0, c->stream>>>(Zc, Yc, N, c->npair, c->dconst);             \
       k_el_contract_mirror<X, T2><<<nbm, 256, 0, c->stream>>>(Zc, Yc, N, c->npair, c->dconst);        \
