@@ -10,10 +10,16 @@
 // A piece goes to whoever is free and nobody waits for a thread that has not
 // begun: after a caller's OpenMP region its threads hold every CPU for a
 // while, a new thread then starts 3 to 4 ms late, and the calling thread does
-// the work alone.
-// Measured, one field read (set), before against now: n = 196 FP64 3.4 (2.0)
-// -> 1.4 (1.4) ms, FP32 3.5 (2.7) -> 0.8 (0.8) ms; n = 260 FP32 21.8 (16.3)
-// -> 1.6 (1.7) ms; n = 36 FP32 21 to 90 -> 20 us.  Chunks: a copy costs about 13 us
+// the work alone.  A helper that lost its CPU in the middle of a piece is
+// waited for.
+// Measured, median of one field read (set) in ms, the runtime's pageable copy
+// (and, for FP32, a conversion through the heap) against this: FP64 n = 148 1.46
+// (0.69) -> 0.68 (0.67), 196 3.5 (2.05) -> 1.41 (1.46), 260 8.0 (4.7) -> 3.1
+// (3.2); FP32 148 1.30 (1.14) -> 0.38 (0.39), 196 3.5 (2.9) -> 0.75 (0.79), 260
+// 21.8 (16.7) -> 1.60 (1.72); n = 36 FP32 21 to 90 -> 20 us.  After an OpenMP
+// region: FP64 196 3.55 (2.0) -> 3.57 (1.6), 260 8.1 (4.7) -> 6.0 (3.55, but one
+// copy in ten 6.5 to 10), FP32 196 7.7 (2.85) -> 1.33 (1.84), 260 29.6 (17) -> 2.7
+// (3.6).  Chunks: a copy costs about 13 us
 // besides its bytes, so 512 KiB pieces reach 21 GB/s, 4 MiB 43 GB/s; more
 // than 4 threads add nothing.
 #include <hip/hip_runtime.h>
@@ -197,7 +203,9 @@ static hipError_t hc_run(hc_job<T> *j) {
 // Pinned memory for a call's slots.  It is taken for the call and given back
 // after it (a copy is over when it returns), so contexts share it: allocating
 // it per context cost an ensemble of 20 a millisecond each.  At most
-// HC_POOL buffers wait between calls; the last context to close frees them.
+// HC_POOL buffers wait between calls, one for each copy that has all its
+// helpers (HC_LIVE / 3), 12 MiB each at most; the last context to close frees
+// them.
 #define HC_POOL 4
 static std::mutex pool_mu;
 static struct {

@@ -81,7 +81,7 @@ struct etd_ctx {
   int Vf_e0, Vif_e0;
   double *DDX, *DDY, *DDZ; /* D / h^2 per axis */
   double *lam;             /* nac x 9 */
-  double *gtmp;            /* 3 x n3 gradient scratch for F2, or CH t */
+  double *gtmp;            /* 3 x n3 scratch: the variable-mobility CH term, the alpha dumps' bytes */
   /* elastic */
   double *Z, *Y;           /* npair x N^3 complex */
   double *E;               /* ring x N^3 */
@@ -91,8 +91,8 @@ struct etd_ctx {
   /* the fields the elastic force acts on: AC fields (ELASTIC = 1) or CH
    * fields (ELASTIC = 2), nel of them from field el_v0; nel = 0 without */
   int nel, el_v0;
-  /* el_mix: more than six variants are transformed as the six strain
-   * components they span (nft = 6 fields instead of nel), see launch_elastic */
+  /* el_mix: more than six variants are transformed as six strains that
+   * span them (nft = 6 fields instead of nel), see launch_elastic */
   int el_mix, nft;
   long long elastic_evals; /* completed elastic evaluations */
   int elastic_fresh;       /* the latest evaluation is of the current fields (adaptive energy test) */

@@ -875,7 +875,7 @@ struct nl_args {
   int P, px, py, pz, bx, by, bz;
   long long bs;
   int bxo, byo, bzo;
-  const double *ev;  // el_mix: the variants' six strain components (E then holds stresses), or null
+  const double *ev;  // el_mix: the variants' components of the six strains (E then holds stresses), or null
 };
 
 // -1 / 0 / +1: the extended coordinate e lies before, in or after the interior
@@ -1092,6 +1092,7 @@ __global__ __launch_bounds__(256) void k_nonlin_ac(const T *__restrict__ u, T *_
 // cells near the faces need is skipped by waves that have none: 238 us, 372
 // us in FP64 (3.8 and 4.9 TB/s of the 30 field passes).  Reading the lagged
 // cells' values field by field made the few waves that have them the longest.
+// It holds every field, so the field batch (nl_batch) means nothing here.
 template <typename T, int FB>
 __global__ __launch_bounds__(256) void k_nonlin_mix(const T *__restrict__ u, T *__restrict__ out,
                                                     const T *__restrict__ sub, const T *__restrict__ E, nl_args a,
@@ -2026,7 +2027,7 @@ __global__ void k_el_pack_boxes(const T *__restrict__ u, typename cplx<T>::t *__
   Z[N3 * r + m] = zz;
 }
 
-// el_mix: the six strain components of a point from every field, one box or
+// el_mix: the components of the six strains at a point from every field, one box or
 // px per axis of edge N (the same addressing)
 template <typename T>
 __global__ __launch_bounds__(256) void k_el_pack_mix(const T *__restrict__ u, typename cplx<T>::t *__restrict__ Z,
@@ -2376,8 +2377,8 @@ void launch_elastic(etd_ctx *c) {
   const int slot0 = (int)(Lbase % c->ring);
   // two-stage FFT: the pack is the forward x pass's input and the unpack the
   // inverse z pass's output
-  // (the fused passes exist only where the two-stage kernel does: N = 16 R2
-  // with an instantiated R2; elsewhere pack, radix passes and unpack)
+  // (the fused passes exist only where the two-stage kernel does, R1 = 16 or
+  // an edge of etd_fft2.hip; elsewhere pack, radix passes and unpack)
   const bool fused = c->fft_variant == 1 && fft2_supported(N) && c->P == 1;
   const double *ev = c->el_mix ? c->dconst->ev : nullptr;
   fft_io io{uel, F.E, c->n, c->g, c->nel, c->ring, slot0, ev};
