@@ -84,92 +84,112 @@ static void c4_from_voigt(const double *C2, double *C4) {
 }
 
 // The six strains E_a that more than six variants are transformed as (el_mix,
-// launch_elastic), unit[9 a + 3 i + j], and every variant's components of
-// them, ev[6 q + a].  Any basis of the symmetric strains gives the same force;
-// this one is orthonormal in the elastic energy averaged over the directions
-// of k, so that what the FP32 fields round in one component weighs as much as
-// in another.  With the strains xx, yy, .. themselves a volume change, which a
-// cubic C makes several times stiffer, was the difference of rounded
-// components: the mixed force of 12 traceless variants at n = 68 was off by
-// 3.0e-7 (rms) against 1.6e-7 of a transform per variant.
-static void strain_basis(const double *C4, const double *eps, int nel, double *unit, double *ev) {
+// launch_elastic): their stresses and energies (k->sig, k->t0), and every
+// variant's components of them (k->ev).  Any basis of the symmetric strains
+// gives the same force; this one is orthonormal in the elastic energy averaged
+// over the directions of k, so that what the fields round in one component
+// weighs as much as in another.  With the strains xx, yy, .. themselves a volume
+// change, which a cubic C makes several times stiffer, was the difference of
+// rounded components: the mixed force of 12 traceless variants at n = 68 was off
+// by 3.0e-7 (rms) against 1.6e-7 of a transform per variant.  In long double, so
+// that each constant is rounded once.
+static void strain_basis(const double *eps, int nel, etd_dev_consts *k) {
+  typedef long double real;
   static const int ij[6][2] = {{0, 0}, {1, 1}, {2, 2}, {1, 2}, {0, 2}, {0, 1}};
-  double M[6][6] = {{0}}, Q[6][6] = {{0}}, e[6][9] = {{0}}, sg[6][9];
+  const double *C4 = k->C4;
+  real M[6][6] = {{0}}, Q[6][6] = {{0}}, e[6][9] = {{0}}, sg[6][9], U[6][6];
   for (int a = 0; a < 6; a++) {  // e: orthonormal as matrices
     const int i = ij[a][0], j = ij[a][1];
-    e[a][3 * i + j] = e[a][3 * j + i] = i == j ? 1.0 : sqrt(0.5);
-    Q[a][a] = 1.0;
+    e[a][3 * i + j] = e[a][3 * j + i] = i == j ? 1.0L : sqrtl(0.5L);
+    Q[a][a] = 1;
     for (int l = 0; l < 9; l++) {
-      sg[a][l] = 0.0;
+      sg[a][l] = 0;
       for (int m = 0; m < 9; m++) sg[a][l] += C4[9 * l + m] * e[a][m];
     }
   }
   // M_ab = sum over directions of e_a : C : e_b - (n sg_a) (C n n)^-1 (sg_b n)
   for (int d = 0; d < 125; d++) {
-    double v[3] = {d % 5 - 2.0, d / 5 % 5 - 2.0, d / 25 - 2.0};
-    const double r = sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
-    if (r == 0.0) continue;
-    double G[3][3], O[3][3], w[6][3];
+    real v[3] = {d % 5 - 2.0L, d / 5 % 5 - 2.0L, d / 25 - 2.0L};
+    const real r = sqrtl(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
+    if (r == 0) continue;
+    real G[3][3], O[3][3], w[6][3];
     for (int i = 0; i < 3; i++) v[i] /= r;
     for (int i = 0; i < 3; i++)
-      for (int k = 0; k < 3; k++) {
-        G[i][k] = 0.0;
+      for (int m = 0; m < 3; m++) {
+        G[i][m] = 0;
         for (int j = 0; j < 3; j++)
-          for (int l = 0; l < 3; l++) G[i][k] += C4[((i * 3 + j) * 3 + k) * 3 + l] * v[j] * v[l];
+          for (int l = 0; l < 3; l++) G[i][m] += C4[((i * 3 + j) * 3 + m) * 3 + l] * v[j] * v[l];
       }
     for (int i = 0; i < 3; i++)  // cofactors, transposed
-      for (int k = 0; k < 3; k++)
-        O[k][i] = G[(i + 1) % 3][(k + 1) % 3] * G[(i + 2) % 3][(k + 2) % 3] -
-                  G[(i + 1) % 3][(k + 2) % 3] * G[(i + 2) % 3][(k + 1) % 3];
-    const double det = G[0][0] * O[0][0] + G[0][1] * O[1][0] + G[0][2] * O[2][0];
+      for (int m = 0; m < 3; m++)
+        O[m][i] = G[(i + 1) % 3][(m + 1) % 3] * G[(i + 2) % 3][(m + 2) % 3] -
+                  G[(i + 1) % 3][(m + 2) % 3] * G[(i + 2) % 3][(m + 1) % 3];
+    const real det = G[0][0] * O[0][0] + G[0][1] * O[1][0] + G[0][2] * O[2][0];
     for (int a = 0; a < 6; a++)
       for (int i = 0; i < 3; i++) w[a][i] = sg[a][3 * i] * v[0] + sg[a][3 * i + 1] * v[1] + sg[a][3 * i + 2] * v[2];
     for (int a = 0; a < 6; a++)
       for (int b = 0; b < 6; b++) {
         for (int l = 0; l < 9; l++) M[a][b] += e[a][l] * sg[b][l];
         for (int i = 0; i < 3; i++)
-          for (int k = 0; k < 3; k++) M[a][b] -= w[a][i] * O[i][k] * w[b][k] / det;
+          for (int m = 0; m < 3; m++) M[a][b] -= w[a][i] * O[i][m] * w[b][m] / det;
       }
   }
-  double big = 0.0;
+  real big = 0;
   bool ok = true;
   for (int a = 0; a < 6; a++)
     for (int b = 0; b <= a; b++) {
-      M[a][b] = M[b][a] = 0.5 * (M[a][b] + M[b][a]);
-      ok = ok && isfinite(M[a][b]);
+      M[a][b] = M[b][a] = (M[a][b] + M[b][a]) / 2;
+      ok = ok && isfinite((double)M[a][b]);
     }
   // Jacobi rotations: the columns of Q become M's eigenvectors
   for (int sweep = 0; ok && sweep < 30; sweep++)
     for (int a = 0; a < 6; a++)
       for (int b = a + 1; b < 6; b++) {
-        if (M[a][b] == 0.0) continue;
-        const double th = (M[b][b] - M[a][a]) / (2.0 * M[a][b]);
-        const double t = (th < 0.0 ? -1.0 : 1.0) / (fabs(th) + sqrt(th * th + 1.0));
-        const double c = 1.0 / sqrt(t * t + 1.0), s = t * c;
-        for (int k = 0; k < 6; k++) {
-          const double x = M[k][a], y = M[k][b];
-          M[k][a] = c * x - s * y, M[k][b] = s * x + c * y;
+        if (M[a][b] == 0) continue;
+        const real th = (M[b][b] - M[a][a]) / (2 * M[a][b]);
+        const real t = (th < 0 ? -1.0L : 1.0L) / (fabsl(th) + sqrtl(th * th + 1));
+        const real c = 1 / sqrtl(t * t + 1), s = t * c;
+        for (int m = 0; m < 6; m++) {
+          const real x = M[m][a], y = M[m][b];
+          M[m][a] = c * x - s * y, M[m][b] = s * x + c * y;
         }
-        for (int k = 0; k < 6; k++) {
-          const double x = M[a][k], y = M[b][k];
-          M[a][k] = c * x - s * y, M[b][k] = s * x + c * y;
+        for (int m = 0; m < 6; m++) {
+          const real x = M[a][m], y = M[b][m];
+          M[a][m] = c * x - s * y, M[b][m] = s * x + c * y;
         }
-        for (int k = 0; k < 6; k++) {
-          const double x = Q[k][a], y = Q[k][b];
-          Q[k][a] = c * x - s * y, Q[k][b] = s * x + c * y;
+        for (int m = 0; m < 6; m++) {
+          const real x = Q[m][a], y = Q[m][b];
+          Q[m][a] = c * x - s * y, Q[m][b] = s * x + c * y;
         }
       }
-  for (int a = 0; a < 6; a++) big = fmax(big, M[a][a]);
+  for (int a = 0; a < 6; a++) big = fmaxl(big, M[a][a]);
+  // E_a = sum_b U_ba e_b, U = Q scaled by 1 / sqrt of the stiffness (1 where the
+  // constants give none: C = 0, not positive)
+  real f[6], E[6][9];
   for (int a = 0; a < 6; a++) {
-    // 1 / sqrt of the stiffness; 1 where the constants give none (C = 0, not positive)
-    const double f = ok && M[a][a] > 1e-8 * big ? sqrt(big / M[a][a]) : 1.0;
+    f[a] = ok && M[a][a] > 1e-8L * big ? sqrtl(big / M[a][a]) : 1.0L;
+    for (int b = 0; b < 6; b++) U[b][a] = f[a] * (ok ? Q[b][a] : a == b ? 1.0L : 0.0L);
     for (int l = 0; l < 9; l++) {
-      unit[9 * a + l] = 0.0;
-      for (int b = 0; b < 6; b++) unit[9 * a + l] += f * (ok ? Q[b][a] : a == b) * e[b][l];
+      E[a][l] = 0;
+      for (int b = 0; b < 6; b++) E[a][l] += U[b][a] * e[b][l];
     }
-    for (int q = 0; q < nel; q++) {  // E_a / f are orthonormal; e and so E_a are symmetric
-      ev[6 * q + a] = 0.0;
-      for (int l = 0; l < 9; l++) ev[6 * q + a] += unit[9 * a + l] / (f * f) * eps[9 * q + l];
+  }
+  for (int a = 0; a < 6; a++) {
+    real S[9];
+    for (int l = 0; l < 9; l++) {
+      S[l] = 0;
+      for (int m = 0; m < 9; m++) S[l] += C4[9 * l + m] * E[a][m];
+      k->sig[9 * a + l] = (double)S[l];
+    }
+    for (int b = 0; b < 6; b++) {
+      real t0 = 0;
+      for (int l = 0; l < 9; l++) t0 += S[l] * E[b][l];
+      k->t0[b * ETD_MAX_VAR + a] = (double)t0;
+    }
+    for (int q = 0; q < nel; q++) {  // E_a / f are orthonormal; the symmetric part of eps, since E_a is symmetric
+      real c = 0;
+      for (int l = 0; l < 9; l++) c += E[a][l] * eps[9 * q + l];
+      k->ev[6 * q + a] = (double)(c / (f[a] * f[a]));
     }
   }
 }
@@ -427,16 +447,9 @@ extern "C" int etd_create(const etd_params *p, const double *Vh, const double *V
     free(tw);
     etd_dev_consts *k = (etd_dev_consts *)calloc(1, sizeof(etd_dev_consts));
     c4_from_voigt(p->C, k->C4);
-    // the transformed fields' eigenstrains: the variants', or six strains
-    // that span them
-    const double *eps = p->eps0;
-    double unit[6 * 9];
-    if (c->el_mix) {
-      strain_basis(k->C4, p->eps0, c->nel, unit, k->ev);
-      eps = unit;
-    }
-    for (int q = 0; q < c->nft; q++) {
-      const double *e = eps + 9 * q;
+    if (c->el_mix) strain_basis(p->eps0, c->nel, k);
+    for (int q = 0; !c->el_mix && q < c->nel; q++) {
+      const double *e = p->eps0 + 9 * q;
       for (int i = 0; i < 3; i++)
         for (int j = 0; j < 3; j++) {
           double s = 0.0;
@@ -445,10 +458,10 @@ extern "C" int etd_create(const etd_params *p, const double *Vh, const double *V
           k->sig[9 * q + i * 3 + j] = s;
         }
     }
-    for (int a = 0; a < c->nft; a++)
-      for (int b = 0; b < c->nft; b++) {
+    for (int a = 0; !c->el_mix && a < c->nel; a++)
+      for (int b = 0; b < c->nel; b++) {
         double t0 = 0.0;
-        const double *ea = eps + 9 * a, *eb = eps + 9 * b;
+        const double *ea = p->eps0 + 9 * a, *eb = p->eps0 + 9 * b;
         for (int i = 0; i < 3; i++)
           for (int j = 0; j < 3; j++)
             for (int kk = 0; kk < 3; kk++)
