@@ -437,10 +437,10 @@ extern "C" int etd_create(const etd_params *p, const double *Vh, const double *V
       HCHK(c, hipMemsetAsync(c->f32.E, 0, sizeof(float) * c->N3 * nE, c->stream));
     }
     double *tw = (double *)malloc(sizeof(double) * 2 * c->Ne);
-    const double pi = 3.14159265358979323846;
-    for (int e = 0; e < c->Ne; e++) {
-      tw[2 * e] = cos(2.0 * pi * e / c->Ne);
-      tw[2 * e + 1] = -sin(2.0 * pi * e / c->Ne);
+    const long double pi = 3.141592653589793238462643383279502884L;
+    for (int e = 0; e < c->Ne; e++) {  // in long double: rounded once
+      tw[2 * e] = (double)cosl(2 * pi * e / c->Ne);
+      tw[2 * e + 1] = (double)-sinl(2 * pi * e / c->Ne);
     }
     HCHK(c, hipMalloc(&c->tw, sizeof(double) * 2 * c->Ne));
     HCHK(c, hipMemcpy(c->tw, tw, sizeof(double) * 2 * c->Ne, hipMemcpyHostToDevice));

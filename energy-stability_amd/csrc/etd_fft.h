@@ -75,6 +75,30 @@ __device__ __forceinline__ void dft_r(double2 *a) {
 template <int R, int SGN>
 __device__ __forceinline__ void dft_any(double2 *a);
 
+// (cos, sin) of 2 pi m / N, rounded once; a constant after unrolling.  The
+// angle is taken within an eighth of a turn and in two parts: formed in one,
+// 2 pi m / N is off by up to 4e-16, which every transform of that length then
+// repeats (cos of a sixth of a turn came out as 0.5 + 1.1e-16).
+template <int N>
+__device__ __forceinline__ double2 turn(int m) {
+  const double pi = 3.14159265358979323846, pi_lo = 1.22464679914735317723e-16;
+  const int q = 4 * m / N % 4, r = 4 * m % N;  // quarter turns, and r / N of one
+  double c, s;
+  if (3 * r == N || 3 * r == 2 * N) {
+    c = 0.86602540378443864676, s = 0.5;
+  } else {
+    const int k = 2 * r <= N ? r : N - r;
+    const double p = pi * k, a = p / (2 * N);
+    const double lo = (fma(-a, (double)(2 * N), p) + fma(pi, (double)k, -p) + pi_lo * k) / (2 * N);
+    c = fma(-lo, sin(a), cos(a)), s = fma(lo, cos(a), sin(a));
+  }
+  if (2 * r > N) {
+    const double t = c;
+    c = s, s = t;
+  }
+  return q == 0 ? make_double2(c, s) : q == 1 ? make_double2(-s, c) : q == 2 ? make_double2(-c, -s) : make_double2(s, -c);
+}
+
 template <int A, int B, int SGN>
 __device__ __forceinline__ void dft_split(double2 *x) {  // size A B, in place, natural order
   double2 y[A][B];
@@ -89,8 +113,8 @@ __device__ __forceinline__ void dft_split(double2 *x) {  // size A B, in place, 
       if (n1 * k2 == 0) {
         y[n1][k2] = t[k2];
       } else {
-        const double ang = 2.0 * 3.14159265358979323846 * (double)(n1 * k2) / (double)(A * B);
-        y[n1][k2] = cmul(t[k2], make_double2(cos(ang), -SGN * sin(ang)));
+        const double2 w = turn<A * B>(n1 * k2);
+        y[n1][k2] = cmul(t[k2], make_double2(w.x, -SGN * w.y));
       }
     }
   }
